@@ -463,6 +463,13 @@ int shard_decode_attn_noalloc(const shard_decode_args* args, void* stream);
  * through it. */
 int shard_kv_reconstruct(const shard_decode_args* args, uint16_t* k_out,
                          uint16_t* v_out, void* stream);
+/* The same with the fp16 segments around the compressed span, the whole of
+ * _ensure_dequant (cache.py:87-124) without its concatenation: k_out / v_out
+ * are (B, G, T, D) fp16 contiguous, T = n_sink + n_comp + n_win + n_stream +
+ * n_dec, rows in that order (sink, compressed, window, stream s_k / s_v,
+ * decode tokens). */
+int shard_kv_rebuild(const shard_decode_args* args, uint16_t* k_out,
+                     uint16_t* v_out, void* stream);
 
 #ifdef __cplusplus
 }

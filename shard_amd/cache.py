@@ -84,6 +84,12 @@ class CacheLayer(CacheLayerMixin):
         if gc is None:
             return
         B = gc["batch"]
+        n_stream = gc.get("stream_n", 0) // B if "k_idx_buf" in gc else 0
+        whole = ops.kv_rebuild(gc, B, n_stream)
+        if whole is not None:
+            self._keys, self._values = whole
+            self._needs_decompress = False
+            return
         k_mid, v_mid = ops.kv_reconstruct(gc, B)
         parts_k = [gc["sink_k"], k_mid, gc["win_k"]]
         parts_v = [gc["sink_v"], v_mid, gc["win_v"]]

@@ -838,22 +838,68 @@ def decode_workspace_bytes(call: DecodeCall) -> int:
     return call.workspace_bytes()
 
 
+def _rebuild_args(fmt, batch: int) -> DecodeArgs:
+    """The compressed-segment fields of a layer for the rebuild entry points:
+    the rank padded to a multiple of 32 where that is at most 256 (zero nibbles
+    and basis columns, which the MFMA rebuild takes), the stored rank
+    otherwise."""
+    _require_gpu(fmt["k_coeffs"])
+    a = DecodeArgs()
+    a.batch, a.n_kv_heads, a.head_dim = batch, fmt["n_kv"], fmt["head_dim"]
+    a.n_comp, a.compress_start = fmt["n_compress"], fmt["compress_start"]
+    padded = 0 < fmt.get("rank_pad", 0) <= 256
+    a.rank = fmt["rank_pad"] if padded else fmt["rank"]
+    a.k_coeffs = fmt["k_coeffs_pad" if padded else "k_coeffs"].data_ptr()
+    a.k_coeff_scale = fmt["k_coeff_scale_pad" if padded else "k_coeff_scale"].data_ptr()
+    a.k_basis = fmt["k_basis_pad" if padded else "k_basis_f16"].data_ptr()
+    a.k_mean, a.inv_freq = fmt["k_mean_f16"].data_ptr(), fmt["inv_freq_dev"].data_ptr()
+    cb = fmt["v_centroids_f16"]  # its own shape: any group and codebook size the Cache takes
+    a.v_codebook, (a.v_codebook_n, a.v_group) = cb.data_ptr(), cb.shape
+    a.v_idx, a.v_ch = fmt["v_indices"].data_ptr(), fmt["v_ch_f16"].data_ptr()
+    return a
+
+
 def kv_reconstruct(fmt, batch: int):
     """Full fp16 K (RoPE re-applied) and V of the compressed segment: (B, G, n, D)."""
     lib = _lib.load()
     dev = fmt["k_coeffs"].device
-    B, G, n, D = batch, fmt["n_kv"], fmt["n_compress"], fmt["head_dim"]
-    q_dummy = torch.empty(B, G * 4, D, dtype=torch.float16, device=dev)
-    call = make_decode_args(q_dummy, fmt, 0, None)
-    cb = fmt["v_centroids_f16"]  # its own shape: any group and codebook size the Cache takes
-    call.args.v_codebook = cb.data_ptr()
-    call.args.v_codebook_n, call.args.v_group = cb.shape
-    call.args.k_coeffs = fmt["k_coeffs"].data_ptr()
-    call.args.k_coeff_scale = fmt["k_coeff_scale"].data_ptr()
-    call.args.k_basis = fmt["k_basis_f16"].data_ptr()
-    call.args.rank = fmt["rank"]
-    k_out = torch.empty(B, G, n, D, dtype=torch.float16, device=dev)
-    v_out = torch.empty(B, G, n, D, dtype=torch.float16, device=dev)
+    k_out = torch.empty(batch, fmt["n_kv"], fmt["n_compress"], fmt["head_dim"], dtype=torch.float16,
+                        device=dev)
+    v_out = torch.empty_like(k_out)
     _lib.check("shard_kv_reconstruct", lib.shard_kv_reconstruct(
-        ctypes.byref(call.args), _p(k_out), _p(v_out), _stream(k_out)))
+        ctypes.byref(_rebuild_args(fmt, batch)), _p(k_out), _p(v_out), _stream(k_out)))
+    return k_out, v_out
+
+
+def kv_rebuild(fmt, batch: int, stream_n: int = 0):
+    """fp16 K and V of the whole layer, (B, G, T, D): sink, compressed span,
+    window, the first stream_n stream rows, then the fp16 decode tokens.  None
+    when a segment is not the contiguous fp16 (B, G, n, D) (stream rows (n, B,
+    G, D)) on the layer's device that the kernel copies: the caller then
+    concatenates."""
+    a = _rebuild_args(fmt, batch)
+    dev, G, D = fmt["k_coeffs"].device, fmt["n_kv"], fmt["head_dim"]
+    total = a.n_comp
+    for name, field, kv in (("n_sink", "sink", ("sink_k", "sink_v")), ("n_win", "win", ("win_k", "win_v")),
+                            ("n_stream", "s", ("k_deq_buf", "v_deq_buf")),
+                            ("n_dec", "dec", ("decode_k", "decode_v"))):
+        stream = field == "s"
+        if (stream_n if stream else kv[0] in fmt) == 0:
+            continue
+        k, v = fmt[kv[0]], fmt[kv[1]]
+        n = stream_n if stream else k.shape[2]
+        shape = (k.shape[0], batch, G, D) if stream else (batch, G, n, D)
+        for t in (k, v):
+            if (t.dtype != torch.float16 or t.device != dev or not t.is_contiguous()
+                    or tuple(t.shape) != shape or (stream and t.shape[0] < n)):
+                return None
+        setattr(a, name, n)
+        setattr(a, field + "_k", k.data_ptr())
+        setattr(a, field + "_v", v.data_ptr())
+        total += n
+    a.dec_stride = a.n_dec
+    k_out = torch.empty(batch, G, total, D, dtype=torch.float16, device=dev)
+    v_out = torch.empty_like(k_out)
+    _lib.check("shard_kv_rebuild", _lib.load().shard_kv_rebuild(
+        ctypes.byref(a), _p(k_out), _p(v_out), _stream(k_out)))
     return k_out, v_out

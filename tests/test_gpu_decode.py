@@ -442,6 +442,77 @@ def test_kv_reconstruct_vq_shapes(cuda, group, n_cent):
     assert np.array_equal(v_got.cpu().numpy().view(np.uint16), v_want.numpy().view(np.uint16))
 
 
+@pytest.mark.parametrize("B,nkv,hd,rank,n_comp,n_stream,n_dec", [
+    (1, 1, 128, 32, 5, 0, 0), (3, 3, 128, 192, 31, 2, 0), (2, 8, 64, 64, 33, 1, 0),
+    (1, 9, 64, 256, 64, 0, 3), (2, 2, 256, 96, 65, 3, 2), (1, 8, 128, 190, 129, 5, 0),
+    (1, 8, 128, 192, 2500, 7, 0)])
+def test_kv_rebuild_edges(cuda, B, nkv, hd, rank, n_comp, n_stream, n_dec):
+    """The MFMA rebuild at the edges of its 32-token tiles, head groups and
+    ranks (190: padded to 192), and the whole layer in one call: the compressed
+    rows within fp16 rounding of the oracle (V bit-exact), the other rows the
+    segments' own, bit for bit, through aligned and unaligned pointers."""
+    import ctypes
+    from shard_amd import _lib, ops
+    gc, inv = random_layer(B=B, nkv=nkv, hd=hd, rank=rank, n_comp=n_comp, n_stream=n_stream,
+                           n_dec=n_dec, seed=rank + n_comp)
+    d = to_device(gc, cuda, inv, nkv=nkv, hd=hd)
+    k_want, v_want = ref.reconstruct_kv(gc, nkv, hd, inv)
+    sk, sv = (d["k_deq_buf"], d["v_deq_buf"]) if n_stream else (None, None)
+
+    def whole(p, mid, stream):
+        parts = [d["sink_" + p], mid.to(cuda), d["win_" + p]]
+        parts += [stream.permute(1, 2, 0, 3)] if n_stream else []
+        return torch.cat(parts + ([d["decode_" + p]] if n_dec else []), 2)
+
+    kw, vw = whole("k", k_want, sk), whole("v", v_want, sv)
+    bits = lambda t: t.cpu().numpy().view(np.uint16)
+
+    def check(k, v):
+        assert k.shape == kw.shape and v.shape == vw.shape
+        assert np.array_equal(bits(v), bits(vw))
+        diff = (k.float() - kw.float()).abs()
+        assert float(diff.max()) <= 2 * 2.0 ** -10   # an ulp of the pre-RoPE value, as above
+        assert float((diff > 0).float().mean()) < 0.02
+        mid = slice(gc["sink_k"].shape[2], gc["sink_k"].shape[2] + n_comp)
+        diff[:, :, mid] = 0
+        assert float(diff.max()) == 0
+
+    k, v = ops.kv_rebuild(d, B, n_stream)
+    check(k, v)
+    k_mid, v_mid = ops.kv_reconstruct(d, B)
+    s0 = gc["sink_k"].shape[2]
+    assert torch.equal(k_mid, k[:, :, s0:s0 + n_comp]) and torch.equal(v_mid, v[:, :, s0:s0 + n_comp])
+    # two bytes past the alignment of the wide accesses: same values
+    odd = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:]
+    a = ops._rebuild_args(d, B)
+    idx, mean = odd(d["v_indices"]), odd(d["k_mean_f16"])
+    a.v_idx, a.k_mean = idx.data_ptr(), mean.data_ptr()
+    ko, vo = odd(k_mid), odd(v_mid)
+    ko.zero_(), vo.zero_()
+    _lib.check("shard_kv_reconstruct", _lib.load().shard_kv_reconstruct(
+        ctypes.byref(a), ko.data_ptr(), vo.data_ptr(), None))
+    torch.cuda.synchronize()
+    assert torch.equal(vo.view_as(v_mid), v_mid)
+    assert float((ko.view_as(k_mid).float() - k_mid.float()).abs().max()) <= 2 * 2.0 ** -10
+
+
+def test_kv_rebuild_non_finite_values(cuda):
+    """V of a layer with infinite, NaN and largest-fp16 channel scales: the
+    rebuilt values are the oracle's, infinities and NaN included."""
+    from shard_amd import ops
+    gc, inv = random_layer(B=1, nkv=4, hd=128, rank=64, n_comp=100, seed=31)
+    ch = gc["v_ch_f16"].view(4, 128)
+    ch[0, 5], ch[1, 7], ch[2] = float("inf"), float("nan"), 65504.0
+    d = to_device(gc, cuda, inv, nkv=4, hd=128)
+    _, v = ops.kv_reconstruct(d, 1)
+    _, want = ref.reconstruct_kv(gc, 4, 128, inv)
+    got, want = v.cpu().numpy(), want.numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert np.array_equal(got.view(np.uint16)[ok], want.view(np.uint16)[ok])
+    assert np.isinf(want).any() and np.isnan(want).any() and np.isfinite(want).any()
+
+
 def test_decode_small_codebook_fused(cuda):
     """A 64-row codebook of 4-value subvectors decodes on the fused kernels
     (padded to 256 rows that no index names) within the fp64 oracle's
