@@ -181,7 +181,9 @@ __device__ __forceinline__ void fwht_lane_stage(float (&x)[E], int l) {
   }
 }
 
-template <int E>
+// RCP: the division by sqrt(d) through its reciprocal (the same values, see
+// div_by_rcp; rows holding a non-finite value divide).
+template <int E, bool RCP = false>
 __device__ __forceinline__ void wave_fwht(float (&x)[E], int d) {
   // d == 64 * E: element i = lane + 64 k; strides 1..32 cross lanes, 64.. cross registers
   const int l = (int)lane_id();
@@ -204,6 +206,17 @@ __device__ __forceinline__ void wave_fwht(float (&x)[E], int d) {
   }
   // torch divides an fp32 tensor by the Python float sqrt(d): fp32(double sqrt)
   const float s = (float)sqrt((double)d);
+  if constexpr (RCP) {
+    bool odd = false;
+#pragma unroll
+    for (int k = 0; k < E; ++k) odd |= !(fabsf(x[k]) < INFINITY);
+    if (__builtin_amdgcn_ballot_w64(odd) == 0) {
+      const float y = div_rn(1.f, s);
+#pragma unroll
+      for (int k = 0; k < E; ++k) x[k] = div_by_rcp(x[k], s, y);
+      return;
+    }
+  }
 #pragma unroll
   for (int k = 0; k < E; ++k) x[k] = div_rn(x[k], s);
 }

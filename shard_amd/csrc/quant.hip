@@ -1470,11 +1470,21 @@ struct StreamIO {
   uint16_t* deq[2];
 };
 
+// Thread i's entry of the LDS codebook: padded to 256 entries no value exceeds.
+__device__ __forceinline__ float codebook_entry(const float* __restrict__ cb_g, int n_codes) {
+  return (int)threadIdx.x < n_codes ? cb_g[threadIdx.x] : INFINITY;
+}
+
 // Quantize row r held by one wave (t = its fp16 values as fp32, lane l holds
-// elements l + 64 k) with the codebook cb (LDS); outputs at row r.
+// elements l + 64 k, sg = their signs) with the codebook cb (LDS, 256 entries);
+// outputs at row r.  A lone wave's chain of dependent operations bounds it
+// (one wave per row, a decode step has a few dozen rows), so the codebook
+// search takes four 4-way steps, the lane's elements side by side, the norm's
+// eight sums meet in scalar registers, and the divisions by the norm and by
+// sqrt(D) go through reciprocals: the same values (div_by_rcp; a row with an
+// infinite norm comes out NaN either way).
 template <int E>
-__device__ __forceinline__ void stream_quant_row(float (&t)[E], int64_t r,
-                                                 const float* __restrict__ signs,
+__device__ __forceinline__ void stream_quant_row(float (&t)[E], int64_t r, const float (&sg)[E],
                                                  const float* cb, int n_codes,
                                                  uint8_t* __restrict__ idx,
                                                  uint16_t* __restrict__ norm,
@@ -1494,29 +1504,46 @@ __device__ __forceinline__ void stream_quant_row(float (&t)[E], int64_t r,
     float v = __shfl(sq[(8 * m) >> 6], (l + 8 * m) & 63, 64);
     acc = add_rn(acc, v);  // meaningful in lanes 0..7 (lane j holds accumulator j)
   }
-  float tot = __shfl(acc, 0, 64);
+  auto lane_val = [](float v, int j) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
+  };
+  float tot = lane_val(acc, 0);
 #pragma unroll
-  for (int j = 1; j < 8; ++j) tot = add_rn(tot, __shfl(acc, j, 64));
-  float n = fmaxf(sqrtf(tot), 1e-8f);
+  for (int j = 1; j < 8; ++j) tot = add_rn(tot, lane_val(acc, j));
+  const float n = fmaxf(sqrtf(tot), 1e-8f), rcp_n = div_rn(1.f, n);
 #pragma unroll
-  for (int k = 0; k < E; ++k) t[k] = mul_sign(div_rn(t[k], n), signs[l + 64 * k]);
-  wave_fwht<E>(t, D);
+  for (int k = 0; k < E; ++k) t[k] = mul_sign(div_by_rcp(t[k], n, rcp_n), sg[k]);
+  wave_fwht<E, true>(t, D);
+  // first i with v <= cb[i] (torch.bucketize, right=False), at most the last
+  // entry: every step keeps the largest of 4 starts whose predecessor is < v
+  int pos[E];
+#pragma unroll
+  for (int k = 0; k < E; ++k) pos[k] = 0;
+#pragma unroll
+  for (int step = 64; step >= 1; step >>= 2) {
+    float c[E][3];
+#pragma unroll
+    for (int k = 0; k < E; ++k)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) c[k][j] = cb[pos[k] + (j + 1) * step - 1];
+#pragma unroll
+    for (int k = 0; k < E; ++k)
+      pos[k] += step * ((c[k][0] < t[k] ? 1 : 0) + (c[k][1] < t[k] ? 1 : 0) + (c[k][2] < t[k] ? 1 : 0));
+  }
+  float cl[E], ci[E];
 #pragma unroll
   for (int k = 0; k < E; ++k) {
-    float v = t[k];
-    int lo = 0, hi = n_codes;  // first i with v <= cb[i] (torch.bucketize, right=False)
-    while (lo < hi) {
-      int mid = (lo + hi) >> 1;
-      if (cb[mid] < v) lo = mid + 1; else hi = mid;
-    }
-    int i = lo < n_codes - 1 ? lo : n_codes - 1;
-    int left = i > 0 ? i - 1 : 0;
-    float dl = fabsf(sub_rn(cb[left], v));
-    float di = fabsf(sub_rn(cb[i], v));
-    const int code = dl < di ? left : i;
-    idx[r * D + l + 64 * k] = (uint8_t)code;
-    res[k] = sub_rn(v, cb[code]);  // QJL residual (streaming.py:69)
-    t[k] = cb[code];
+    pos[k] = min(pos[k], n_codes - 1);
+    cl[k] = cb[max(pos[k] - 1, 0)];
+    ci[k] = cb[pos[k]];
+  }
+#pragma unroll
+  for (int k = 0; k < E; ++k) {
+    const float v = t[k];
+    const bool left = fabsf(sub_rn(cl[k], v)) < fabsf(sub_rn(ci[k], v));
+    idx[r * D + l + 64 * k] = (uint8_t)(left ? max(pos[k] - 1, 0) : pos[k]);
+    t[k] = left ? cl[k] : ci[k];
+    res[k] = sub_rn(v, t[k]);  // QJL residual (streaming.py:69)
   }
   const uint16_t nh = f2h(n);
   if (l == 0) norm[r] = nh;
@@ -1554,11 +1581,11 @@ __device__ __forceinline__ void stream_quant_row(float (&t)[E], int64_t r,
   }
   if (deq) {
     // reference dequant: fp16(fp16(hadamard(cb[idx] (+ qjl)) * signs) * fp16 norm)
-    wave_fwht<E>(t, D);
+    wave_fwht<E, true>(t, D);
     const float nf = h2f(nh);
 #pragma unroll
     for (int k = 0; k < E; ++k)
-      deq[r * D + l + 64 * k] = f2h_opaque(h2f(f2h(mul_sign(t[k], signs[l + 64 * k]))) * nf);
+      deq[r * D + l + 64 * k] = f2h_opaque(h2f(f2h(mul_sign(t[k], sg[k]))) * nf);
   }
 }
 
@@ -1569,17 +1596,21 @@ __global__ void k_stream_quant(const StreamIO io, int64_t rows,
   constexpr int D = 64 * E;
   const int job = blockIdx.y;
   __shared__ float cb[256];
-  for (int i = threadIdx.x; i < n_codes; i += blockDim.x) cb[i] = cb_g[i];
-  __syncthreads();
+  const float cbv = codebook_entry(cb_g, n_codes);
   const int l = (int)lane_id();
   const int w = threadIdx.x >> 6;
-  int64_t r = (int64_t)blockIdx.x * (blockDim.x >> 6) + w;
-  if (r >= rows) return;  // no block-level barrier below this point
+  const int64_t r = (int64_t)blockIdx.x * (blockDim.x >> 6) + w;
   const uint16_t* __restrict__ x = io.x[job];
-  float t[E];
+  float t[E], sg[E];
 #pragma unroll
-  for (int k = 0; k < E; ++k) t[k] = h2f(x[r * D + l + 64 * k]);
-  stream_quant_row<E>(t, r, signs, cb, n_codes, io.idx[job], io.norm[job], io.qsign[job],
+  for (int k = 0; k < E; ++k) {
+    t[k] = h2f(x[min(r, rows - 1) * D + l + 64 * k]);
+    sg[k] = signs[l + 64 * k];
+  }
+  cb[threadIdx.x] = cbv;
+  __syncthreads();
+  if (r >= rows) return;  // no block-level barrier below this point
+  stream_quant_row<E>(t, r, sg, cb, n_codes, io.idx[job], io.norm[job], io.qsign[job],
                       io.qscale[job], io.deq[job]);
 }
 
@@ -1587,28 +1618,31 @@ __global__ void k_stream_quant(const StreamIO io, int64_t rows,
 // Decode-step front end: RoPE of q and k with transformers' fp16 arithmetic
 // (apply_rotary_pos_emb: q * cos + rotate_half(q) * sin, each product and the
 // sum rounded to fp16 as torch's half ops do), then the new token's k and v
-// quantized into the stream (as k_stream_quant).  One wave per row: rows
-// [0, B H) are q rows (-> q_out), the next B G rows k, the last B G rows v.
+// quantized into the stream (as k_stream_quant).  One wave per row, 4 rows per
+// workgroup: rows [0, B H) are q rows (-> q_out), the next B G rows k, the
+// last B G rows v.  Every load a row needs (its values, phases, signs, the
+// codebook, the stream row) goes out before the barrier.  Launched back to
+// back at batch 1 (32 + 16 rows of 128): 3.20 us against 4.21 with the row's
+// loads behind the codebook's barrier, one 8-step search per element and IEEE
+// division sequences; one row per 64-thread workgroup 3.57.
 // E >= 2 and even: the RoPE pair (d, d + D / 2) of element l + 64 k is element
 // l + 64 (k + E / 2) of the same lane.
 // ---------------------------------------------------------------------------
 template <int E>
-__device__ __forceinline__ void rope_row(float (&t)[E], const uint16_t* __restrict__ c,
-                                         const uint16_t* __restrict__ sn) {
+__device__ __forceinline__ void rope_row(float (&t)[E], const float (&c)[E], const float (&sn)[E]) {
   const int l = (int)lane_id();
   float o[E];
 #pragma unroll
   for (int k = 0; k < E; ++k) {
-    const int d = l + 64 * k;
     float rot;  // rotate_half
     if constexpr (E == 1) {  // head_dim 64: the partner dim is 32 lanes away
-      const float pt = __shfl_xor(t[0], 32);
+      const float pt = xor_lane<32>(t[0]);
       rot = l < 32 ? -pt : pt;
     } else {
       rot = k < E / 2 ? -t[k + E / 2] : t[k - E / 2];
     }
-    const float a = h2f(f2h(mul_rn(t[k], h2f(c[d]))));
-    const float b = h2f(f2h(mul_rn(rot, h2f(sn[d]))));
+    const float a = h2f(f2h(mul_rn(t[k], c[k])));
+    const float b = h2f(f2h(mul_rn(rot, sn[k])));
     o[k] = h2f(f2h(add_rn(a, b)));
   }
 #pragma unroll
@@ -1616,56 +1650,52 @@ __device__ __forceinline__ void rope_row(float (&t)[E], const uint16_t* __restri
 }
 
 template <int E>
-__global__ void k_rope_stream(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kx,
-                              const uint16_t* __restrict__ vx, const uint16_t* __restrict__ cosv,
-                              const uint16_t* __restrict__ sinv, int64_t cs_stride, int B,
-                              int H, int G, uint16_t* __restrict__ q_out, const StreamIO io,
-                              const float* __restrict__ signs, const float* __restrict__ cb_g,
-                              int n_codes, const int32_t* __restrict__ row_dev, int row_cap) {
+__global__ __launch_bounds__(256)
+void k_rope_stream(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kx,
+                   const uint16_t* __restrict__ vx, const uint16_t* __restrict__ cosv,
+                   const uint16_t* __restrict__ sinv, int64_t cs_stride, int B, int H, int G,
+                   uint16_t* __restrict__ q_out, const StreamIO io,
+                   const float* __restrict__ signs, const float* __restrict__ cb_g, int n_codes,
+                   const int32_t* __restrict__ row_dev, int row_cap) {
   constexpr int D = 64 * E;
   __shared__ float cb[256];
-  for (int i = threadIdx.x; i < n_codes; i += blockDim.x) cb[i] = cb_g[i];
-  __syncthreads();
   const int l = (int)lane_id();
-  const int64_t r = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int64_t nq = (int64_t)B * H, nk = (int64_t)B * G;
-  if (r >= nq + 2 * nk) return;  // no block-level barrier below this point
-  float t[E];
-  if (r < nq) {
-    const int64_t b = r / H;
+  const uint32_t nq = (uint32_t)B * H, nk = (uint32_t)B * G;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const uint32_t r = min(wave, nq + 2 * nk - 1);      // waves past the last row repeat it
+  const int job = r < nq ? -1 : r < nq + nk ? 0 : 1;  // -1: q, 0: k, 1: v
+  const uint32_t rr = job < 0 ? r : r - nq - (job ? nk : 0);
+  const uint16_t* __restrict__ x = job < 0 ? q : job == 0 ? kx : vx;
+  const float cbv = codebook_entry(cb_g, n_codes);
+  // with row_dev the outputs are the buffers' bases and the token's row comes
+  // from device memory (a captured graph replays one launch for every decode
+  // step); a row outside [0, row_cap) writes nothing
+  const int64_t row = row_dev ? *row_dev : 0;
+  float t[E], c[E], sn[E], sg[E];
+  const int64_t b = rr / (uint32_t)(job < 0 ? H : G);
 #pragma unroll
-    for (int k = 0; k < E; ++k) t[k] = h2f(q[r * D + l + 64 * k]);
-    rope_row<E>(t, cosv + b * cs_stride, sinv + b * cs_stride);
+  for (int k = 0; k < E; ++k) {
+    t[k] = h2f(x[(int64_t)rr * D + l + 64 * k]);
+    c[k] = h2f(cosv[b * cs_stride + l + 64 * k]);
+    sn[k] = h2f(sinv[b * cs_stride + l + 64 * k]);
+    sg[k] = signs[l + 64 * k];
+  }
+  cb[threadIdx.x] = cbv;
+  __syncthreads();  // no barrier below this point
+  if (wave > r) return;
+  if (job < 1) rope_row<E>(t, c, sn);
+  if (job < 0) {
 #pragma unroll
-    for (int k = 0; k < E; ++k) q_out[r * D + l + 64 * k] = f2h(t[k]);
+    for (int k = 0; k < E; ++k) q_out[(int64_t)r * D + l + 64 * k] = f2h(t[k]);
     return;
   }
-  const int job = r < nq + nk ? 0 : 1;  // 0: k, 1: v
-  const int64_t rr = r - nq - job * nk;
-  const uint16_t* __restrict__ x = job == 0 ? kx : vx;
-#pragma unroll
-  for (int k = 0; k < E; ++k) t[k] = h2f(x[rr * D + l + 64 * k]);
-  if (job == 0) rope_row<E>(t, cosv + (rr / G) * cs_stride, sinv + (rr / G) * cs_stride);
-  uint8_t* idx = io.idx[job];
-  uint16_t* norm = io.norm[job];
+  if (row_dev && (row < 0 || row >= row_cap)) return;
   uint8_t* qsign = io.qsign[job];
-  uint16_t* qscale = io.qscale[job];
   uint16_t* deq = io.deq[job];
-  if (row_dev) {
-    // the outputs are the buffers' bases and the token's row comes from device
-    // memory (a captured graph replays one launch for every decode step); a
-    // row outside [0, row_cap) writes nothing
-    const int64_t row = *row_dev;
-    if (row < 0 || row >= row_cap) return;
-    idx += row * nk * D;
-    norm += row * nk;
-    if (qsign) {
-      qsign += row * nk * D;
-      qscale += row * nk;
-    }
-    if (deq) deq += row * nk * D;
-  }
-  stream_quant_row<E>(t, rr, signs, cb, n_codes, idx, norm, qsign, qscale, deq);
+  stream_quant_row<E>(t, rr, sg, cb, n_codes, io.idx[job] + row * nk * D, io.norm[job] + row * nk,
+                      qsign ? qsign + row * nk * D : nullptr,
+                      qsign ? io.qscale[job] + row * nk : nullptr,
+                      deq ? deq + row * nk * D : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -2186,6 +2216,7 @@ static int rope_stream_launch(const uint16_t* q, const uint16_t* k, const uint16
                        {k_qsign, v_qsign}, {k_qscale, v_qscale}, {k_deq, v_deq}};
   hipStream_t s = (hipStream_t)stream;
   const int64_t rows = (int64_t)batch * (n_q_heads + 2 * n_kv_heads);
+  if (rows > INT32_MAX) return SHARD_ERR_SHAPE;
   const dim3 grid((unsigned)((rows + 3) / 4));
   switch (hd) {
     case 64: hipLaunchKernelGGL(k_rope_stream<1>, grid, dim3(256), 0, s, q, k, v, cos, sin, cos_stride, batch, n_q_heads, n_kv_heads, q_rope, io, signs, codebook, n_codes, row_dev, row_cap); break;
