@@ -8,8 +8,9 @@
 //     of compressed tokens, walked 32 tokens at a time.  The 4 waves share each
 //     tile: wave P rebuilds rows of the 16 RoPE pairs [16 P, 16 P + 16) (basis
 //     operand in VGPRs), the partial scores meet in LDS, then a shared online
-//     softmax and VQ value sum.  The last split of each head first runs the
-//     extra tokens (at most 2048) into one more partial row per query head.
+//     softmax and VQ value sum.  The extra tokens (at most 2048) run on
+//     workgroups of their own, 128 tokens each, one more partial row per
+//     query head and workgroup.
 //   k_decode_tok (token-tiled)  grid = n_splits * n_kv * query groups * B,
 //     512-thread workgroups, one per CU, 1, 2 or 4 query heads per workgroup;
 //     the kv head's basis operand image sits in LDS and each wave takes whole
@@ -65,8 +66,8 @@ constexpr int kTokMaxRank = 256;            // the token-tiled kernel (the row-s
 #define SHARD_SPLIT_PER_XCD 1
 #endif
 constexpr bool kSplitPerXcd = SHARD_SPLIT_PER_XCD;
-// Row-split launches in two classes whose (batch row, kv head) groups fill
-// the 8 XCDs evenly put every split of a group on one XCD and run the group's
+// Row-split launches whose (batch row, kv head) groups fill the 8 XCDs evenly
+// put every split of a group on one XCD and run the group's
 // merge workgroups there too, so the merge reads the partial rows that XCD's
 // L2 wrote (8K, batch 1: 13.86 -> 13.51 us).  SHARD_KV_XCD=0 keeps the split
 // order of the other launches.
@@ -98,11 +99,14 @@ __device__ __forceinline__ int extras_now(const ExtraSegs& s) {
 struct SplitParams {
   int32_t B, H, G, rank, n_comp, cstart, pos_q, n_splits;
   const int64_t* pos_q_dev;  // when set, pos_q is read from device memory
-  // Token ranges: splits [0, n_first) cover `chunk` tokens each, the others
-  // `chunk2` (two_class: the first and the second workgroup of each CU).
-  int32_t chunk, chunk2, n_first, two_class;
-  int32_t nsp;   // partial rows per (batch row, query head): n_splits (+1 with extra tokens)
-  ExtraSegs xs;  // processed by the last split of each head before its compressed tiles
+  // The n_splits workgroups of a (batch row, kv head): n_xs run the extra
+  // tokens, as splits [x_at, x_at + n_xs); the others, in order,
+  // run the compressed tiles.  The first n_first tile splits take `tiles`
+  // tiles, the first `more` of them one more, the later ones tiles2 and more2
+  // likewise (two_class: the first and the second workgroup of each CU).
+  int32_t n_xs, x_at, x_wave;  // x_wave: extra tokens per wave, a multiple of 4
+  int32_t n_first, tiles, more, tiles2, more2, two_class;
+  ExtraSegs xs;
   const uint16_t* q;
   const float* inv_freq;
   const uint8_t* coef;
@@ -117,8 +121,8 @@ struct SplitParams {
   float* ws_m;
   float* ws_l;
   float* ws_acc;
-  // kv_xcd (two_class launches whose (batch row, kv head) groups fill the 8
-  // XCDs evenly): every split of a group on one XCD
+  // kv_xcd (launches whose (batch row, kv head) groups fill the 8 XCDs
+  // evenly): every split of a group on one XCD
   int32_t kv_xcd;
 };
 
@@ -365,31 +369,43 @@ constexpr bool kSplitBias = SHARD_SPLIT_BIAS;
 // MI355X (19.2 vs 18.4 us at 8K) and is kept as a build option only.
 constexpr int kTG = SHARD_DECODE_TG;
 static_assert(kTG == 1 || kTG == 2, "SHARD_DECODE_TG must be 1 or 2");
+// Extra tokens per wave of an extra-token workgroup: kXLong, or kXShort (a
+// shorter value loop) for up to kXFew tokens where the workgroups that adds
+// take none from the tiles and none more per CU.  At 1K with 132 extra tokens
+// a 33rd split per head would no longer fit one workgroup per CU: 14.6 us per
+// layer-step against 13.3.  Within the rule the two are close (1.5K: 14.8 us
+// against 15.0 with 78 extra tokens, 15.1 against 14.7 with 132).
+constexpr int kXFew = 256, kXShort = 16, kXLong = 32;
 
-// Extra tokens (sink, window, decode, stream; fp16 rows) of kv head g, run by
-// the last split workgroup of the head before its compressed tiles, with NW
-// waves.  Per pass of 32 NW tokens: scores on MFMA (rows = the kGQA query
-// heads, k = head dims, columns = the wave's 32 tokens), online softmax per
-// head (wave h < kGQA owns head h), values accumulated lane-per-dim pair.
-// Writes partial row n_splits of each query head, in the plain (not rotated)
-// basis.
+// Extra tokens (sink, window, decode, stream; fp16 rows) xi XT .. xi XT + XT of
+// kv head g, XT = NW x_wave, on a workgroup of their own: scores on MFMA (rows =
+// the kGQA query heads, k = head dims, columns = the wave's 32 tokens),
+// softmax per head (wave h < kGQA owns head h), values accumulated
+// lane-per-dim pair.  Writes partial row `split` of each query head, in the
+// plain (not rotated) basis; empty (m = -inf) when the call has fewer tokens.
+// A pass takes about 14K clocks whatever it holds, the time of several
+// compressed tiles: run by one workgroup before its tiles, pass after pass, it
+// was the critical path of short contexts and of streams past 60 tokens (per
+// layer-step of append, split and merge at batch 1, 132 extra tokens: 2K 17.5
+// -> 14.9 us, 3.5K 17.5 -> 16.0, 8K 19.0 -> 18.2; 8K with 868: 18.1,
+// where the token-tiled kernel takes 20.9).  Tried and not kept: V rows in
+// 16-byte loads, 16 lanes a row (15.1 at 2K: the sums of 16 row groups meet in
+// LDS instead of 4).
 template <int NW>
 struct XtLds {
   float xsc[kGQA][32 * NW];     // scores of the pass (base 2)
   float xpw[32 * NW][kGQA];     // softmax numerators, [token][head]
   float2 xred[NW][kGQA][64];    // per-wave value sums
-  float xal[kGQA];              // rescale of the running sums
 };
 
 template <int NW>
-__device__ __forceinline__ void decode_extras_tail(const SplitParams& p, const int g, const int b,
-                                                   XtLds<NW>& L) {
-  constexpr int XT = 32 * NW;  // tokens per pass
-  constexpr int XV = XT / 64;  // softmax values per lane
+__device__ __forceinline__ void decode_extras(const SplitParams& p, const int g, const int b,
+                                              const int split, const int xi, XtLds<NW>& L) {
+  constexpr int XV = 32 * NW / 64;        // softmax values per lane
+  const int tw = p.x_wave, XT = NW * tw;  // tokens per wave, per workgroup
   auto& xsc = L.xsc;
   auto& xpw = L.xpw;
   auto& xred = L.xred;
-  auto& xal = L.xal;
 
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, hh = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -409,9 +425,10 @@ __device__ __forceinline__ void decode_extras_tail(const SplitParams& p, const i
   float2 acc[kGQA];
 #pragma unroll
   for (int h = 0; h < kGQA; ++h) acc[h] = make_float2(0.f, 0.f);
-
-  for (int x0 = 0; x0 < n_x; x0 += XT) {
-    const int xt = min(x0 + 32 * w + col, n_x - 1);  // clamped: rows past n_x are masked
+  const int x0 = xi * XT;
+  if (x0 < n_x) {
+    const bool mine = col < tw && x0 + tw * w + col < n_x;
+    const int xt = min(x0 + tw * w + min(col, tw - 1), n_x - 1);  // clamped: other rows are masked
     int mpos;
     const uint16_t* krow = extra_row(p.xs, p.B, p.G, p.n_comp, b, g, xt, false, &mpos);
     const uint16_t* vrow = extra_row(p.xs, p.B, p.G, p.n_comp, b, g, xt, true, &mpos);
@@ -423,6 +440,7 @@ __device__ __forceinline__ void decode_extras_tail(const SplitParams& p, const i
     const uint64_t vb = (uint64_t)vrow;
 #pragma unroll
     for (int t = 0; t < 32; ++t) {
+      if (t % 4 == 0 && t >= tw) break;
       const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)vb, t);
       const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(vb >> 32), t);
       vx[t] = ld_global_u32((((uint64_t)hi << 32) | lo) + 4 * lane);
@@ -431,12 +449,11 @@ __device__ __forceinline__ void decode_extras_tail(const SplitParams& p, const i
 #pragma unroll
     for (int st = 0; st < 8; ++st) sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(Aq[st], Bk[st], sacc, 0, 0, 0);
     if (hh == 0) {
-      const bool valid = x0 + 32 * w + col < n_x;
 #pragma unroll
-      for (int i = 0; i < kGQA; ++i) xsc[i][32 * w + col] = valid ? sacc[i] * sc + madd : -INFINITY;
+      for (int i = 0; i < kGQA; ++i) xsc[i][32 * w + col] = mine ? sacc[i] * sc + madd : -INFINITY;
     }
     __syncthreads();
-    if (w < kGQA) {  // wave w: online softmax of head w over the pass
+    if (w < kGQA) {  // wave w: softmax of head w
       float s[XV];
       float mx = -INFINITY;
 #pragma unroll
@@ -444,27 +461,20 @@ __device__ __forceinline__ void decode_extras_tail(const SplitParams& p, const i
         s[k] = xsc[w][lane + 64 * k];
         mx = fmaxf(mx, s[k]);
       }
-      const float m_new = fmaxf(m_run, wave64_reduce(mx, OpMax()));
-      const float al = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
+      m_run = wave64_reduce(mx, OpMax());
       float ps = 0.f;
 #pragma unroll
       for (int k = 0; k < XV; ++k) {
-        const float pk = s[k] == -INFINITY ? 0.f : fast_exp2(s[k] - m_new);
+        const float pk = s[k] == -INFINITY ? 0.f : fast_exp2(s[k] - m_run);
         ps += pk;
         xpw[lane + 64 * k][w] = pk;
       }
-      l_run = l_run * al + wave64_reduce(ps, OpAdd());
-      m_run = m_new;
-      if (lane == 0) xal[w] = al;
+      l_run = wave64_reduce(ps, OpAdd());
     }
     __syncthreads();
-    const float4 al4 = *(const float4*)xal;
-    acc[0].x *= al4.x; acc[0].y *= al4.x;
-    acc[1].x *= al4.y; acc[1].y *= al4.y;
-    acc[2].x *= al4.z; acc[2].y *= al4.z;
-    acc[3].x *= al4.w; acc[3].y *= al4.w;
 #pragma unroll
     for (int t = 0; t < 32; ++t) {
+      if (t % 4 == 0 && t >= tw) break;
       const float4 pw = *(const float4*)&xpw[32 * w + t][0];
       const half2v hv = __builtin_bit_cast(half2v, vx[t]);
       const float v0 = (float)hv[0], v1 = (float)hv[1];
@@ -486,7 +496,7 @@ __device__ __forceinline__ void decode_extras_tail(const SplitParams& p, const i
       t.x += a.x;
       t.y += a.y;
     }
-    const int64_t widx = ((int64_t)b * p.H + g * kGQA + h) * p.nsp + p.n_splits;
+    const int64_t widx = ((int64_t)b * p.H + g * kGQA + h) * p.n_splits + split;
     *(float2*)(p.ws_acc + widx * kHD + 2 * lane) = t;
     if (lane == 0) {
       p.ws_m[widx] = m_run;
@@ -533,19 +543,21 @@ void k_decode_split(const SplitParams p) {
   // of every CU with the first 256 workgroups and the second slot with the
   // next 256.  The older workgroup of a CU gets issue priority, so splits
   // [0, n_first) go to the first class with longer chunks and the second class
-  // gets shorter ones; both then finish together.  Each class holds half the
-  // splits of every (batch row, kv head).
+  // gets shorter ones and the extra tokens; both then finish together.  Each
+  // class holds half the splits of every (batch row, kv head).
   const int HG = p.G;
   const int bid = blockIdx.x;
   int hg, split, b;
   if (p.kv_xcd) {
     // every workgroup of a (batch row, kv head) group on one XCD (block id
-    // mod 8): group x + 8 gi on XCD x, its splits of each class in one run
+    // mod 8): group x + 8 gi on XCD x, its splits (two_class: of each class)
+    // in one run
     const int L = blockIdx.y * gridDim.x + bid;  // dispatch order
-    const int c = L >> 8, j = L & 255;
+    const int c = p.two_class ? L >> 8 : 0, j = p.two_class ? L & 255 : L;
+    const int per = p.two_class ? p.n_first : p.n_splits;
     const int r = j >> 3;
-    const int grp_i = (j & 7) + 8 * (r / p.n_first);
-    split = c * p.n_first + r % p.n_first;
+    const int grp_i = (j & 7) + 8 * (r / per);
+    split = c * per + r % per;
     b = grp_i / HG;
     hg = grp_i % HG;
   } else if (p.two_class) {
@@ -567,11 +579,11 @@ void k_decode_split(const SplitParams p) {
     }
     b = blockIdx.y;
   }
-  // The last split of each head runs the extra tokens first (its compressed
-  // chunk is shorter by their cost), so their cold loads overlap the other
-  // workgroups' set-up instead of trailing the kernel.
   __shared__ __align__(16) XtLds<4 * TG> xt;
-  if (split == p.n_splits - 1 && p.xs.n_x > 0) decode_extras_tail<4 * TG>(p, hg, b, xt);
+  if (split >= p.x_at && split < p.x_at + p.n_xs) {  // whole workgroup
+    decode_extras<4 * TG>(p, hg, b, split, split - p.x_at, xt);
+    return;
+  }
 
   // ---- loads that feed LDS and the q operand go out first: the first barrier
   // waits for these only, not for the tile and basis loads behind them.
@@ -588,23 +600,13 @@ void k_decode_split(const SplitParams p) {
       q_hi[jj] = *(const uint2*)(qv + d0 + 64);
     }
   }
-  const int t_begin = split < p.n_first ? split * p.chunk
-                                         : p.n_first * p.chunk + (split - p.n_first) * p.chunk2;
-  int t_end = t_begin + (split < p.n_first ? p.chunk : p.chunk2);
-  if (t_end > p.n_comp) t_end = p.n_comp;
-  if (t_end <= t_begin) {
-    // no compressed tokens (a last split that only holds the extra tokens):
-    // the empty partial row is m = -inf, l = 0, acc = 0; skip the set-up
-    if (tid < 64 * NQ) {
-      const int64_t widx = ((int64_t)b * p.H + hg * NQ + wv) * p.nsp + split;
-      *(float2*)(p.ws_acc + widx * kHD + 2 * lane) = make_float2(0.f, 0.f);
-      if (lane == 0) {
-        p.ws_m[widx] = -INFINITY;
-        p.ws_l[widx] = 0.f;
-      }
-    }
-    return;
-  }
+  const int ts = split < p.x_at ? split : split - p.n_xs;  // tile split
+  const bool cls2 = ts >= p.n_first;
+  const int ti = cls2 ? ts - p.n_first : ts;
+  const int tn = cls2 ? p.tiles2 : p.tiles, tm = cls2 ? p.more2 : p.more;
+  const int t_begin =
+      kTile * ((cls2 ? p.n_first * p.tiles + p.more : 0) + ti * tn + min(ti, tm));
+  const int t_end = min(t_begin + kTile * (tn + (ti < tm ? 1 : 0)), p.n_comp);
 
   // ---- first iteration's loads go out before the setup work.  Token indices
   // are clamped to the chunk (no divergent loads); rows past the chunk end get
@@ -615,7 +617,7 @@ void k_decode_split(const SplitParams p) {
   const int vG = tid & 31;
   const int vts = tid >> 5;
   const uint8_t* vidx_b = p.vidx + (((int64_t)b * p.G + hg) * p.n_comp) * 32 + vG;
-  const int t_last = t_end > t_begin ? t_end - 1 : t_begin;
+  const int t_last = t_end - 1;
   auto load_tile = [&](int t0, uint32_t (&cw_)[KS], uint32_t (&vc_)[VT]) {
     const int tc = min(t0 + kTile * grp + col, t_last);
     load_coef<KS>(coef_b + (int64_t)tc * coef_row_bytes, true, cw_);
@@ -623,7 +625,7 @@ void k_decode_split(const SplitParams p) {
     for (int m = 0; m < VT; ++m) vc_[m] = vidx_b[(int64_t)min(t0 + VT * vts + m, t_last) * 32];
   };
   uint32_t cwA[KS], vcA[VT], cwB[KS], vcB[VT];
-  if (t_begin < t_end) load_tile(t_begin, cwA, vcA);
+  load_tile(t_begin, cwA, vcA);
 
   // ---- per-layer constant operands: coalesced 16-byte loads
   half8 Ab[KS + 1];
@@ -837,7 +839,7 @@ void k_decode_split(const SplitParams p) {
   if (tid < NQ * TT) {
     const float l = TT == 64 ? wave64_reduce(l_part, OpAdd()) : half32_reduce(l_part, OpAdd());
     if (tid % TT == 0) {
-      const int64_t widx = ((int64_t)b * p.H + hg * NQ + tid / TT) * p.nsp + split;
+      const int64_t widx = ((int64_t)b * p.H + hg * NQ + tid / TT) * p.n_splits + split;
       p.ws_m[widx] = m_run;
       p.ws_l[widx] = l;
     }
@@ -865,7 +867,7 @@ void k_decode_split(const SplitParams p) {
     float x0 = rv.x * (float)chh[0], x1 = rv.y * (float)chh[1];
     fwht128_pairs(x0, x1);
     const int qh = hg * NQ + wv;
-    *(float2*)(p.ws_acc + (((int64_t)b * p.H + qh) * p.nsp + split) * kHD + 2 * lane) = make_float2(x0, x1);
+    *(float2*)(p.ws_acc + (((int64_t)b * p.H + qh) * p.n_splits + split) * kHD + 2 * lane) = make_float2(x0, x1);
   }
 }
 
@@ -1544,8 +1546,9 @@ void k_decode_tok(const TokParams p) {
 // shape.  Automatic choice by the work per CU: the token-tiled kernel has the
 // higher tile throughput but a longer set-up, so it takes over from 9
 // head-tiles per CU (measured on MI355X, row-split vs token-tiled, us per
-// call: batch 1 x 8K (7.9 per CU) 14.5-14.6 vs 14.8; 1 x 10K (9.9) 16.2 vs
-// 15.3; 1 x 12K 18.0 vs 17.7; 2 x 8K 20.5 vs 17.9; 1 x 16K 19.4-19.8 vs 17.8).
+// layer-step with append and merge: batch 1 x 8K (7.9 per CU) 17.9 vs 20.1
+// with 268 extra tokens, 20.2 vs 28.4 with 1,968; 1 x 10K (9.9) 19.2 vs 19.2;
+// 1 x 12K 20.8 vs 19.7; 2 x 6K 20.6 vs 19.9; 1 x 16K 22.5 vs 22.2).
 constexpr int kTokMinHeadTilesPerCU = 9;
 
 inline int device_cus() {
@@ -1563,6 +1566,19 @@ inline int device_cus() {
 
 inline int64_t n_extra(const shard_decode_args* a) {
   return (int64_t)a->n_sink + a->n_win + a->n_dec + a->n_stream;
+}
+
+inline ExtraSegs extra_segs(const shard_decode_args* a) {
+  ExtraSegs x;
+  x.sink_k = a->sink_k; x.sink_v = a->sink_v;
+  x.win_k = a->win_k; x.win_v = a->win_v;
+  x.dec_k = a->dec_k; x.dec_v = a->dec_v;
+  x.s_k = a->s_k; x.s_v = a->s_v;
+  x.n_sink = a->n_sink; x.n_win = a->n_win; x.n_dec = a->n_dec;
+  x.dec_stride = a->dec_stride; x.n_stream = a->n_stream;
+  x.n_x = (int32_t)n_extra(a);
+  x.n_stream_dev = a->n_stream_dev;
+  return x;
 }
 
 // The token-tiled kernel's kv heads: head_dim-64 layers run their kv heads in
@@ -1597,32 +1613,66 @@ inline bool split_supported(const shard_decode_args* a) {
          a->rank % 32 == 0 && a->rank <= 192 && n_extra(a) <= kMaxExtra;
 }
 
-// The row-split kernel runs every extra token in its last split, one pass of
-// 128 after another; beyond this many the token-tiled kernel, which spreads
-// them over splits, is faster (measured at 8K: 18.6 vs 18.8 us with 268 extra
-// tokens, 23.3 vs 21.9 with 468, 34.3 vs 22.7 with 1,068).
-constexpr int kRowSplitMaxExtraAuto = 256;
-
 // kernel = 1 asks for the row-split kernel; a call it cannot take (query
 // groups other than 4, more than kMaxExtra extra tokens: the reference appends
 // stream tokens without limit, cache.py:156-181) runs on the token-tiled one.
 inline bool use_tok(const shard_decode_args* a) {
   if (a->kernel == 2) return true;
   if (a->kernel == 1) return !split_supported(a);
-  if (!split_supported(a) || n_extra(a) > kRowSplitMaxExtraAuto) return true;
+  if (!split_supported(a)) return true;
   const int64_t tiles = (int64_t)((a->n_comp + kTile - 1) / kTile) * a->n_kv_heads * a->batch;
   return tiles >= (int64_t)kTokMinHeadTilesPerCU * device_cus();
 }
 
-// Row-split kernel: splits per (batch row, kv head), two workgroups per CU.
-inline int split_count(const shard_decode_args* a) {
-  const int max_useful = (a->n_comp + kTile - 1) / kTile;
-  int want = a->n_splits > 0 ? a->n_splits
-                             : (kTG == 1 ? 2 : 1) * device_cus() / (a->n_kv_heads * a->batch);
-  if (want > max_useful) want = max_useful;
-  if (want < 1) want = 1;
-  if (want > kMaxSplits) want = kMaxSplits;
-  return want;
+// Row-split kernel: the workgroups of a (batch row, kv head).
+struct RowPlan {
+  int n_t, n_xs, n_splits;  // tile splits, extra-token splits, both
+  int n_first, tiles, more, tiles2, more2, two_class, x_at, x_wave;
+};
+
+// Two workgroups per CU in all; the extra tokens take some of them and the
+// compressed tiles the others, as evenly as whole tiles allow.
+inline RowPlan row_plan(const shard_decode_args* a) {
+  RowPlan w;
+  const int n_tiles = (a->n_comp + kTile - 1) / kTile;
+  const int heads = a->n_kv_heads * a->batch, cus = device_cus();
+  const int all = (kTG == 1 ? 2 : 1) * cus / heads;
+  auto plan_extras = [&](int x_wave) {
+    const int x_wg = 4 * kTG * x_wave;
+    w.x_wave = x_wave;
+    w.n_xs = (int)((n_extra(a) + x_wg - 1) / x_wg);
+    w.n_t = std::max(1, std::min({a->n_splits > 0 ? a->n_splits : all - w.n_xs, n_tiles, kMaxSplits}));
+  };
+  plan_extras(kXLong);
+  if (n_extra(a) <= kXFew) {
+    const int n_t = w.n_t, per_cu = ((w.n_t + w.n_xs) * heads + cus - 1) / cus;
+    plan_extras(kXShort);
+    if (w.n_t != n_t || ((w.n_t + w.n_xs) * heads + cus - 1) / cus != per_cu) plan_extras(kXLong);
+  }
+  w.n_splits = w.n_t + w.n_xs;
+  w.n_first = w.n_t;
+  w.tiles = n_tiles / w.n_t;
+  w.more = n_tiles % w.n_t;
+  w.tiles2 = w.more2 = w.two_class = 0;
+  w.x_at = 0;  // the extra tokens' workgroups take longest: dispatched first
+  const int half = w.n_splits / 2, rest = w.n_t - half;
+  // the class split assumes 256 CUs (two classes of 256 workgroups)
+  if (kTG == 1 && kSplitBias && device_cus() == 256 &&
+      (int64_t)w.n_splits * a->n_kv_heads * a->batch == 512 && w.n_splits % 2 == 0 &&
+      32 % a->n_kv_heads == 0 && n_tiles >= 2 * w.n_splits && rest > 0) {
+    const int ta = (97 * half + 64 * n_tiles) / (100 * half);  // round(0.47 + 0.64 n_tiles / half)
+    const int left = n_tiles - half * ta;
+    if (ta >= 1 && left >= rest) {
+      w.n_first = half;
+      w.tiles = ta;
+      w.more = 0;
+      w.tiles2 = left / rest;
+      w.more2 = left % rest;
+      w.two_class = 1;
+      w.x_at = w.n_t;  // the last workgroups of the second class
+    }
+  }
+  return w;
 }
 
 // Token-tiled kernel: the split count and the cost units per split.
@@ -1690,14 +1740,7 @@ int decode_attn_tok(const shard_decode_args* a, float* ws, hipStream_t s) {
   tp.QG = a->n_q_heads / tp.G / nq;
   tp.cstart = a->compress_start;
   tp.n_ct = pl.n_ct; tp.n_xt = pl.n_xt; tp.n_splits = pl.ns; tp.per_u = pl.per_u;
-  tp.xs.sink_k = a->sink_k; tp.xs.sink_v = a->sink_v;
-  tp.xs.win_k = a->win_k; tp.xs.win_v = a->win_v;
-  tp.xs.dec_k = a->dec_k; tp.xs.dec_v = a->dec_v;
-  tp.xs.s_k = a->s_k; tp.xs.s_v = a->s_v;
-  tp.xs.n_sink = a->n_sink; tp.xs.n_win = a->n_win; tp.xs.n_dec = a->n_dec;
-  tp.xs.dec_stride = a->dec_stride; tp.xs.n_stream = a->n_stream;
-  tp.xs.n_x = (int32_t)n_extra(a);
-  tp.xs.n_stream_dev = a->n_stream_dev;
+  tp.xs = extra_segs(a);
   tp.q = a->q; tp.inv_freq = a->inv_freq; tp.coef = a->k_coeffs;
   tp.op = (const uint4*)a->prep;
   tp.rope = (const float2*)((const char*)a->prep + (size_t)tp.G * 4 * (a->rank / 16 + 1) * 64 * sizeof(uint4));
@@ -1767,8 +1810,7 @@ size_t shard_decode_attn_workspace(const shard_decode_args* a) {
     const TokPlan pl = tok_plan(a);
     return (size_t)a->batch * a->n_q_heads * pl.ns * (kHD + 2) * sizeof(float);
   }
-  const int nsp = split_count(a) + (n_extra(a) > 0 ? 1 : 0);
-  return (size_t)a->batch * a->n_q_heads * nsp * (kHD + 2) * sizeof(float);
+  return (size_t)a->batch * a->n_q_heads * row_plan(a).n_splits * (kHD + 2) * sizeof(float);
 }
 
 }  // extern "C"
@@ -1796,60 +1838,26 @@ static int decode_attn_check(const shard_decode_args* a) {
 static int decode_attn_run(const shard_decode_args* a, void* workspace, hipStream_t s) {
   if (use_tok(a)) return decode_attn_tok(a, (float*)workspace, s);
 
-  const int n_x = (int)n_extra(a);
-  const int ns = split_count(a);
-  const int nsp = ns + (n_x > 0 ? 1 : 0);
+  const RowPlan pl = row_plan(a);
   float* ws = (float*)workspace;
-  const int64_t nm = (int64_t)a->batch * a->n_q_heads * nsp;
+  const int64_t nm = (int64_t)a->batch * a->n_q_heads * pl.n_splits;
   SplitParams sp;
   sp.B = a->batch; sp.H = a->n_q_heads; sp.G = a->n_kv_heads; sp.rank = a->rank;
   sp.n_comp = a->n_comp; sp.cstart = a->compress_start; sp.pos_q = a->pos_q;
   sp.pos_q_dev = a->pos_q_dev;
-  sp.n_splits = ns;
-  // Compressed tiles per split, in whole 32-token tiles.  The last split of
-  // each head also runs the extra tokens (an extra token costs about half a
-  // compressed one), so the tiles are spread over the splits as if there were
-  // n_x / 64 more of them and the last split takes what remains.
-  const int n_tiles = (a->n_comp + kTile - 1) / kTile;
-  const int x_cost = (n_x + 63) / 64;
-  const int cap = n_tiles + x_cost;
-  const int chunk_tiles = (cap + ns - 1) / ns;
-  sp.chunk = ((chunk_tiles + kTG - 1) / kTG) * kTG * kTile;
-  sp.chunk2 = sp.chunk;
-  sp.n_first = ns;
-  sp.two_class = 0;
-  const int half = ns / 2;
-  // the class split and both block orders assume 256 CUs (two classes of 256 workgroups)
-  if (kTG == 1 && kSplitBias && device_cus() == 256 && (int64_t)ns * a->n_kv_heads * a->batch == 512 &&
-      ns % 2 == 0 && 32 % a->n_kv_heads == 0 && n_tiles >= 2 * ns) {
-    // first class: ta tiles per split, second class: tb (the last split also
-    // runs the extra tokens, counted as x_cost tiles)
-    const int ta = (97 * half + 64 * cap) / (100 * half);  // round(0.47 + 0.64 cap / half)
-    const int tb = (cap - half * ta + half - 1) / half;
-    if (ta >= 1 && tb >= 1) {
-      sp.chunk = ta * kTile;
-      sp.chunk2 = tb * kTile;
-      sp.n_first = half;
-      sp.two_class = 1;
-    }
-  }
-  sp.nsp = nsp;
-  sp.xs.sink_k = a->sink_k; sp.xs.sink_v = a->sink_v;
-  sp.xs.win_k = a->win_k; sp.xs.win_v = a->win_v;
-  sp.xs.dec_k = a->dec_k; sp.xs.dec_v = a->dec_v;
-  sp.xs.s_k = a->s_k; sp.xs.s_v = a->s_v;
-  sp.xs.n_sink = a->n_sink; sp.xs.n_win = a->n_win; sp.xs.n_dec = a->n_dec;
-  sp.xs.dec_stride = a->dec_stride; sp.xs.n_stream = a->n_stream; sp.xs.n_x = n_x;
-  sp.xs.n_stream_dev = a->n_stream_dev;
+  sp.n_splits = pl.n_splits; sp.n_xs = pl.n_xs; sp.x_at = pl.x_at; sp.x_wave = pl.x_wave;
+  sp.n_first = pl.n_first; sp.tiles = pl.tiles; sp.more = pl.more;
+  sp.tiles2 = pl.tiles2; sp.more2 = pl.more2; sp.two_class = pl.two_class;
+  sp.xs = extra_segs(a);
   sp.q = a->q; sp.inv_freq = a->inv_freq; sp.coef = a->k_coeffs;
   sp.op = (const uint4*)a->prep;
   sp.rope = (const float2*)((const char*)a->prep + shard_decode_prepare_op_bytes(a->n_kv_heads, a->rank));
   sp.vidx = a->v_idx; sp.vcb = a->v_codebook; sp.vch = a->v_ch;
   sp.mask = a->mask; sp.mask_stride = a->mask_stride; sp.n_sink = a->n_sink;
   sp.ws_m = ws; sp.ws_l = ws + nm; sp.ws_acc = ws + 2 * nm;
-  sp.kv_xcd = SHARD_KV_XCD && sp.two_class && (a->batch * a->n_kv_heads) % 8 == 0;
+  sp.kv_xcd = SHARD_KV_XCD && (a->batch * a->n_kv_heads) % 8 == 0;
 
-  dim3 grid((unsigned)(ns * a->n_kv_heads), (unsigned)a->batch);
+  dim3 grid((unsigned)(pl.n_splits * a->n_kv_heads), (unsigned)a->batch);
   switch (a->rank / 16) {
     case 2: hipLaunchKernelGGL((k_decode_split<2, kTG>), grid, dim3(256 * kTG), 0, s, sp); break;
     case 4: hipLaunchKernelGGL((k_decode_split<4, kTG>), grid, dim3(256 * kTG), 0, s, sp); break;
@@ -1860,7 +1868,7 @@ static int decode_attn_run(const shard_decode_args* a, void* workspace, hipStrea
     default: return SHARD_ERR_SHAPE;
   }
   SHARD_LAUNCH_CHECK("shard_decode_attn row-split kernel");
-  return launch_merge(a, ws, nsp, s, sp.kv_xcd ? kGQA : 0);
+  return launch_merge(a, ws, pl.n_splits, s, sp.kv_xcd ? kGQA : 0);
 }
 
 // ---- scratch of shard_decode_attn_noalloc: the partial rows (m, l, acc) of

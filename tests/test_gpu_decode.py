@@ -404,6 +404,38 @@ def test_decode_config5_layer_full_size(cuda):
     assert err <= TOL_ABS and cos >= TOL_COS, (err, cos)
 
 
+@pytest.mark.parametrize("B,nkv,n_comp,n_stream,planned", [
+    (1, 8, 1000, 61, 61),     # 129 extra tokens: one past a workgroup's 128
+    (1, 8, 1500, 60, 60),     # 128, in two short passes
+    (1, 2, 40, 1, 1900),      # planned for 16 workgroups of extra tokens, 15 of them empty
+    (1, 8, 8124, 190, 400),   # two classes, four workgroups per head for the extra tokens
+    (2, 8, 2100, 0, 0),
+    (16, 8, 300, 5, 5)])
+def test_row_split_extra_workgroups(cuda, B, nkv, n_comp, n_stream, planned):
+    """The row-split kernel's workgroups of extra tokens at the edges of their
+    128- and 64-token passes, planned for more stream rows than the device
+    count holds (empty partial rows), against the fp64 oracle."""
+    from shard_amd import ops
+    gc, inv = random_layer(B=B, nkv=nkv, n_comp=n_comp, n_stream=max(n_stream, 1), seed=n_comp)
+    d = to_device(gc, cuda, inv, nkv=nkv)
+    if not n_stream:
+        gc.pop("stream_n")
+    for p in "kv":  # rows past the count: NaN, so a read of them shows
+        buf = torch.full((max(planned, 1), B, nkv, 128), float("nan"), dtype=torch.float16, device=cuda)
+        buf[:n_stream] = d[p + "_deq_buf"][:n_stream]
+        d[p + "_deq_buf"] = buf
+    q = torch.randn(B, 4 * nkv, 1, 128, generator=torch.Generator().manual_seed(5)).half()
+    pos_q = 4 + n_comp + 64 + n_stream
+    want = exact.decode_attention(q.numpy(), gc, nkv, pos_q, inv.numpy())
+    count = torch.tensor([n_stream], dtype=torch.int32, device=cuda)
+    call = ops.make_decode_args(q.to(cuda).reshape(B, -1, 128), d, pos_q, None, stream_n=planned,
+                                stream_n_dev=count if planned else None)
+    call.args.kernel = 1
+    got = ops.decode_attn(call).cpu().float().numpy().reshape(want.shape)
+    err, cos = compare(got, want)
+    assert err <= TOL_ABS and cos >= TOL_COS, (err, cos)
+
+
 @pytest.mark.parametrize("rank,nkv,hd", [(160, 8, 128), (320, 8, 128), (512, 4, 128), (320, 8, 64)])
 def test_kv_reconstruct(cuda, rank, nkv, hd):
     """Unfused fp16 reconstruction (_ensure_dequant): V bit-exact, K within fp16
