@@ -471,6 +471,18 @@ int shard_kv_reconstruct(const shard_decode_args* args, uint16_t* k_out,
 int shard_kv_rebuild(const shard_decode_args* args, uint16_t* k_out,
                      uint16_t* v_out, void* stream);
 
+/* The `top` largest eigenvalues (descending) and their unit eigenvectors
+ * (evecs: (top, n) row-major) of the symmetric float64 matrix a (n, n), n <=
+ * 1024, which is overwritten: the PCA basis of a layer's key covariance
+ * (svd_lowrank of cache.py:376-378, exactly and deterministically).
+ * Householder tridiagonalization, Sturm multisection, twisted factorizations.
+ * Vectors of nearly equal eigenvalues (closer than about 1e-6 of the largest)
+ * are not reorthogonalized, and non-finite input gives non-finite output:
+ * check V V^T and the residual before use. */
+size_t shard_eigh_top_workspace(int32_t n);
+int shard_eigh_top(double* a, int32_t n, int32_t top, double* evals, double* evecs,
+                   void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

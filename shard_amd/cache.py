@@ -15,8 +15,8 @@ CacheLayer: 64-292):
                           (_ensure_dequant, cache.py:87-124; HIP reconstruct)
 The compression's per-token work runs in HIP kernels of libshard_hip.so (undo
 RoPE and centring, projection, int4 chain, Hadamard and VQ assignment, k-means
-update); torch computes the column mean and the covariance GEMM of the fp32
-rows, and the host a float64 eigendecomposition of the (p, p) covariance.
+update) and in the float64 eigensolver of the (p, p) covariance; torch computes
+the column mean and the covariance GEMM of the fp32 rows.
 CPU tensors are rejected.
 """
 import torch
@@ -598,24 +598,76 @@ def _eigh_top(cov_host: torch.Tensor, rank: int):
     return evecs.flip(1)[:, :rank].float(), evals.flip(0)[:rank].clamp(min=0.0).float()
 
 
-def pca_basis_cov(cov: torch.Tensor, rank: int):
-    """Top-`rank` eigenvectors of a (p, p) covariance and their eigenvalues, by
-    a float64 symmetric eigendecomposition on the host (deterministic)."""
-    evecs, evals = _eigh_top(cov.double().cpu(), rank)
-    return evecs.to(cov.device), evals.to(cov.device)
-
-
 _host_pool = None
 
 
 def _host_worker():
-    """One background thread for host work that overlaps the GPU (the PCA
-    eigendecomposition runs there while the V codec's kernels run)."""
+    """One background thread for host work beside the caller's (the launches of
+    the PCA eigendecomposition, while the V codec's are issued)."""
     global _host_pool
     if _host_pool is None:
         import concurrent.futures
         _host_pool = concurrent.futures.ThreadPoolExecutor(max_workers=1, thread_name_prefix="shard-host")
     return _host_pool
+
+
+# Bounds an eigensolve on the GPU has to meet (float64 sums of the float32
+# basis it gives are not affected below them): orthogonality of the vectors,
+# residual relative to the largest eigenvalue.
+_EIG_ORTH, _EIG_RESID = 1e-8, 1e-10
+
+
+class _EigJob:
+    """The top-`rank` eigenpairs of a (p, p) covariance, solved on a side
+    stream while the caller's stream goes on: shard_eigh_top in float64 (6.6 ms
+    at p = 1024, most of it the 1,023 launches of the tridiagonalization, which
+    a background thread issues; LAPACK on the host took 50 to 200 ms), checked
+    for orthogonality and residual.  A layer that misses the bounds (clustered
+    or zero eigenvalues, a non-finite covariance) or is larger than the kernel
+    takes goes to the host's float64 eigh, errors included."""
+
+    def __init__(self, cov: torch.Tensor, rank: int):
+        self.cov, self.rank = cov.detach(), rank
+        self.future = None
+        p = cov.shape[0]
+        if not cov.is_cuda or not 2 <= p <= ops.EIGH_MAX or rank < 1:
+            return
+        self.main = torch.cuda.current_stream(cov.device)
+        self.side = torch.cuda.Stream(cov.device)
+        self.side.wait_stream(self.main)
+        self.cov.record_stream(self.side)
+        self.future = _host_worker().submit(self._solve)
+
+    @torch.no_grad()
+    def _solve(self):
+        with torch.cuda.device(self.cov.device), torch.cuda.stream(self.side):
+            cov = self.cov.double()
+            evals, evecs = ops.eigh_top(cov, self.rank)
+            gram = evecs @ evecs.t().contiguous()
+            gram.diagonal().sub_(1.0)
+            vt = evecs.t().contiguous()
+            resid = (cov @ vt - vt * evals).abs().max() / evals[0].abs()
+            return evecs, torch.cat([torch.stack([gram.abs().max(), resid]), evals])
+
+    def result(self):
+        """(basis (p, rank) fp32 on the device, eigenvalues (rank) fp32)."""
+        if self.future is not None:
+            evecs, stat = self.future.result()
+            self.main.wait_stream(self.side)
+            evecs.record_stream(self.main)
+            stat.record_stream(self.main)
+            host_stat = stat.cpu()
+            if host_stat[0] <= _EIG_ORTH and host_stat[1] <= _EIG_RESID:  # False for NaN
+                return evecs.float().t(), host_stat[2:].clamp(min=0.0).float()
+        basis, eig = _eigh_top(self.cov.double().cpu(), self.rank)
+        return basis.to(self.cov.device), eig
+
+
+def pca_basis_cov(cov: torch.Tensor, rank: int):
+    """Top-`rank` eigenvectors of a (p, p) covariance and their eigenvalues, by
+    a float64 symmetric eigendecomposition (deterministic)."""
+    basis, eig = _EigJob(cov, rank).result()
+    return basis, eig.to(cov.device)
 
 
 def pca_basis(centered: torch.Tensor, rank: int):
@@ -624,7 +676,7 @@ def pca_basis(centered: torch.Tensor, rank: int):
     niter=24) (cache.py:376-378).  The reference's randomized subspace iteration
     converges to this subspace; here it is computed exactly and
     deterministically: the fp32 covariance X^T X / n on the GPU (one GEMM), then
-    a float64 symmetric eigendecomposition of the (p, p) matrix on the host."""
+    a float64 symmetric eigendecomposition of the (p, p) matrix."""
     n = centered.shape[0]
     return pca_basis_cov((centered.t() @ centered) / n, rank)
 
@@ -661,9 +713,8 @@ def compress_layer(cache: Cache, k_full: torch.Tensor, v_full: torch.Tensor, li:
         basis = cache._basis_override.get(li)
     eig_job = None
     if basis is None:
-        # the host eigendecomposition overlaps the V codec's GPU work below
-        cov_host = _covariance(centered).double().cpu()
-        eig_job = _host_worker().submit(_eigh_top, cov_host, rank)
+        # the eigendecomposition runs beside the V codec's work below
+        eig_job = _EigJob(_covariance(centered), rank)
     else:
         basis = basis.to(dev, torch.float32)[:, :rank]
         eig = _column_energy(centered, basis)
@@ -674,7 +725,7 @@ def compress_layer(cache: Cache, k_full: torch.Tensor, v_full: torch.Tensor, li:
     centroids, idx = ops.kmeans(x, cache._v_vq_codebook_size, n_iter=30, seed=42)
     del x
     if eig_job is not None:
-        basis, eig = (t.to(dev) for t in eig_job.result())
+        basis, eig = eig_job.result()
     budget = max(64, int(p_dim * 16 / cache._k_target_cr))
     alloc = host.dp_bit_allocation(eig, budget)
     keep = sum(1 for b in alloc if b > 0)

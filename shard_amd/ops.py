@@ -290,6 +290,27 @@ class VqTable:
         return centroids.dim() == 2 and centroids.shape[1] == 4 and k % 32 == 0 and 0 < k <= 256
 
 
+EIGH_MAX = 1024  # the largest order shard_eigh_top takes
+
+
+def eigh_top(a: torch.Tensor, top: int):
+    """The `top` largest eigenvalues (descending) and eigenvectors ((top, n)
+    rows) of the symmetric float64 matrix a (n, n), n <= EIGH_MAX; a is left as
+    it was.  Not reorthogonalized within clusters: callers check the result."""
+    _require_gpu(a)
+    if a.dtype != torch.float64 or a.dim() != 2 or a.shape[0] != a.shape[1]:
+        raise TypeError("eigh_top: a must be a square float64 matrix")
+    lib = _lib.load()
+    n = a.shape[0]
+    work = a.clone(memory_format=torch.contiguous_format)
+    evals = torch.empty(top, dtype=torch.float64, device=a.device)
+    evecs = torch.empty(top, n, dtype=torch.float64, device=a.device)
+    ws = _workspace(lib.shard_eigh_top_workspace(n), a.device)
+    _lib.check("shard_eigh_top", lib.shard_eigh_top(
+        _p(work), n, top, _p(evals), _p(evecs), _p(ws), ws.numel(), _stream(a)))
+    return evals, evecs
+
+
 def vq_undecided_rows(ws: torch.Tensor, n: int) -> int:
     """Rows that the last table assignment of n rows into workspace ws left to
     the all-centroid scan: the per-wave counts at the workspace's start (one

@@ -314,3 +314,37 @@ def test_compress_rank_above_256(cuda):
     diff = (k_got.cpu().float() - k_want.float()).abs()
     print(f"[compress rank 320] rebuilt K max |diff| {float(diff.max()):.3e}", flush=True)
     assert float(diff.max()) <= 2 * 2.0 ** -10 * max(1.0, float(k_want.float().abs().max()))
+
+
+@pytest.mark.parametrize("n,top,rows", [(2, 2, 9), (63, 63, 200), (64, 5, 200), (65, 65, 40),
+                                        (257, 192, 2000), (1023, 30, 3000), (1024, 192, 193)])
+def test_eigh_top_matches_host_eigh(cuda, n, top, rows):
+    """shard_eigh_top against the host's float64 eigh at the edges of its
+    64-column groups and 4-row workgroups, full and rank-deficient (rows below
+    n, where only the nonzero eigenvalues are asked for): eigenvalues within a
+    few n ulps of the largest, vectors orthogonal, residual at rounding."""
+    from shard_amd import ops
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(rows, n, generator=g, dtype=torch.float64)
+    x *= torch.exp(-torch.arange(n) / (0.1 * n + 8))
+    c = x.T @ x / rows
+    top = min(top, rows - 1)
+    w, v = (t.cpu() for t in ops.eigh_top(c.to(cuda), top))
+    want = torch.linalg.eigvalsh(c).flip(0)[:top]
+    eps = 2.0 ** -52 * n * float(want[0])
+    assert float((w - want).abs().max()) <= 4 * eps
+    assert float((c @ v.T - v.T * w).abs().max()) <= 4 * eps
+    gap = float((want[:-1] - want[1:]).min()) if top > 1 else float(want[0])
+    assert float((v @ v.T - torch.eye(top, dtype=torch.float64)).abs().max()) <= max(1e-12, 4 * eps / gap)
+
+
+def test_eig_job_hands_clusters_and_bad_input_to_the_host(cuda):
+    """Equal eigenvalues (whose vectors shard_eigh_top does not orthogonalize),
+    a zero covariance, NaN and an order beyond the kernel's give what the
+    host's eigh gives."""
+    from shard_amd.cache import _EigJob, _eigh_top
+    for c in (torch.eye(96), torch.zeros(64, 64), torch.eye(1030), torch.full((64, 64), float("nan"))):
+        basis, eig = _EigJob(c.to(cuda), 20).result()
+        want, eig_want = _eigh_top(c.double(), 20)
+        assert torch.equal(basis.cpu().nan_to_num(7.0), want.nan_to_num(7.0))
+        assert torch.equal(eig.cpu().nan_to_num(7.0), eig_want.nan_to_num(7.0))
