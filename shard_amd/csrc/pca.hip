@@ -437,6 +437,170 @@ void k_pca_project_rope(const uint16_t* __restrict__ K, int n_kv, int seq, int s
   }
 }
 
+// The undone operand of ROWS rows from row0 on, in the fragment order above,
+// into LDS (rows of 128 n_kv + 8 halves).
+template <int ROWS, int NT>
+__device__ __forceinline__ void undo_rows(const uint16_t* __restrict__ K, int n_kv, int seq, int start,
+                                          int n_comp, int64_t m, const float2* __restrict__ phases,
+                                          int64_t row0, uint16_t* as) {
+  constexpr int UB = 3;
+  // unit = (row, head, 8 pairs): its 16 dims in, two fragments out; UB units'
+  // loads go out together
+  const int b0 = (int)(row0 / n_comp), t0 = (int)(row0 - (int64_t)b0 * n_comp);
+  const int last_row = m - row0 < ROWS ? (int)(m - row0) - 1 : ROWS - 1;
+  const int units = ROWS * n_kv * 8, tid = threadIdx.x, stride = n_kv * 128 + 8;
+  for (int u0 = tid; u0 < units; u0 += UB * NT) {
+    uint4 l4[UB], h4[UB];
+    float4 ph[UB][4];
+    int at[UB];
+#pragma unroll
+    for (int i = 0; i < UB; ++i) {
+      const int u = u0 + i * NT;
+      const uint32_t uu = u < units ? u : tid;
+      const int q8 = uu & 7;
+      const uint32_t rg = uu >> 3, lr = rg / (uint32_t)n_kv;
+      const int g = rg - lr * n_kv;
+      int b = b0, t = t0 + min((int)lr, last_row);  // rows past m: never stored
+      while (t >= n_comp) {
+        t -= n_comp;
+        ++b;
+      }
+      const uint16_t* kp = K + (((int64_t)b * n_kv + g) * seq + start + t) * 128 + 8 * q8;
+      l4[i] = *(const uint4*)kp;
+      h4[i] = *(const uint4*)(kp + 64);
+      const float4* pp = (const float4*)(phases + (int64_t)t * kRopePairs + 8 * q8);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ph[i][e] = pp[e];
+      // 8 q8 = 32 ph + 16 j + 8 hh: k position 64 (2 g + ph) + 16 (2 j + o) + 8 hh
+      at[i] = lr * stride + 128 * g + 64 * (q8 >> 2) + 32 * ((q8 >> 1) & 1) + 8 * (q8 & 1);
+    }
+#pragma unroll
+    for (int i = 0; i < UB; ++i) {
+      const uint32_t lw[4] = {l4[i].x, l4[i].y, l4[i].z, l4[i].w};
+      const uint32_t hw[4] = {h4[i].x, h4[i].y, h4[i].z, h4[i].w};
+      half8 f[2];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float4 c2 = ph[i][e >> 1];
+        const float cs = e & 1 ? c2.z : c2.x, sn = e & 1 ? c2.w : c2.y;
+        const float l = h2f((uint16_t)(lw[e >> 1] >> (16 * (e & 1))));
+        const float h = h2f((uint16_t)(hw[e >> 1] >> (16 * (e & 1))));
+        // undo_rope: k cos - rotate_half(k) sin, rotate_half = [-hi, lo] (k_k_prepare's arithmetic)
+        f[e >> 2][e & 3] = (half_t)__fadd_rn(__fmul_rn(l, cs), __fmul_rn(h, sn));
+        f[e >> 2][4 + (e & 3)] = (half_t)__fsub_rn(__fmul_rn(h, cs), __fmul_rn(l, sn));
+      }
+      if (u0 + i * NT < units) {
+        *(half8*)(as + at[i]) = f[0];
+        *(half8*)(as + at[i] + 16) = f[1];
+      }
+    }
+  }
+}
+
+// The same product, 32 RB rows and all columns per workgroup: the undone
+// operand of the rows (all k, the fragment order above) goes to LDS once, then
+// wave j multiplies it with column block j of Btp straight from L2, 8 k-steps
+// ahead, with no barrier in the loop.  Each output's MFMA sequence is the
+// kernel's above, so the results are the same bits.  It spreads m rows over two
+// to four times as many workgroups and undoes each key once instead of twice;
+// bound by the basis fragments (32 lines of 128 bytes per load, two loads'
+// worth each), so many rows stay with the kernel above (pca_rope_few).
+constexpr int kFewHalves = 80 * 1024;  // the whole 160 KB: these launches put one workgroup on a CU
+
+template <int NB32, int RB>
+__global__ __launch_bounds__(64 * (NB32 < 4 ? 4 : NB32))
+void k_pca_rope_rows(const uint16_t* __restrict__ K, int n_kv, int seq, int start, int n_comp,
+                     int64_t m, const float2* __restrict__ phases,
+                     const uint16_t* __restrict__ Btp, const float* __restrict__ bias,
+                     float* __restrict__ C, int64_t ldc) {
+  constexpr int NT = 64 * (NB32 < 4 ? 4 : NB32);
+  constexpr int ROWS = 32 * RB, RING = 8;
+  __shared__ __align__(16) uint16_t as[kFewHalves];  // [ROWS][k + 8]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hh = lane >> 5;
+  const int k = n_kv * 128, stride = k + 8;
+  const int64_t row0 = (int64_t)blockIdx.x * ROWS;
+  const uint16_t* bcol = Btp + ((int64_t)32 * (w < NB32 ? w : 0) + col) * k + 8 * hh;
+  half8 bc[RING], bn[RING];
+#pragma unroll
+  for (int d = 0; d < RING; ++d) bc[d] = *(const half8*)(bcol + 16 * d);  // k >= 128
+  undo_rows<ROWS, NT>(K, n_kv, seq, start, n_comp, m, phases, row0, as);
+  __syncthreads();
+  if (w >= NB32) return;
+  float16v acc[RB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i) acc[i] = {};
+  const uint16_t* arow = as + col * stride + 8 * hh;
+  const int nk = k / 16;  // a multiple of 8
+  auto round = [&](int s0, const half8 (&cur)[RING], half8 (&nxt)[RING]) {
+    const int sn = s0 + RING < nk ? s0 + RING : 0;  // the last round's are not used
+#pragma unroll
+    for (int d = 0; d < RING; ++d) nxt[d] = *(const half8*)(bcol + 16 * (sn + d));
+    __builtin_amdgcn_sched_group_barrier(0x020, RING, 0);  // the next round's loads first
+#pragma unroll
+    for (int d = 0; d < RING; ++d)
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+            *(const half8*)(arow + 32 * i * stride + 16 * (s0 + d)), cur[d], acc[i], 0, 0, 0);
+  };
+  for (int s0 = 0; s0 < nk; s0 += 2 * RING) {
+    round(s0, bc, bn);
+    if (s0 + RING < nk) round(s0 + RING, bn, bc);
+  }
+  const float bz = bias ? bias[32 * w + col] : 0.f;
+#pragma unroll
+  for (int i = 0; i < RB; ++i) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int64_t rr = row0 + 32 * i + 8 * (e >> 2) + 4 * hh + (e & 3);
+      if (rr < m) C[rr * ldc + 32 * w + col] = acc[i][e] - bz;
+    }
+  }
+}
+
+// The same product for few rows: one 32 x 32 block of C per workgroup, both
+// operands whole in LDS (k <= 1,216), one wave's MFMA chain; the same bits.
+__global__ __launch_bounds__(256)
+void k_pca_rope_block(const uint16_t* __restrict__ K, int n_kv, int seq, int start, int n_comp,
+                      int64_t m, const float2* __restrict__ phases,
+                      const uint16_t* __restrict__ Btp, const float* __restrict__ bias,
+                      float* __restrict__ C, int64_t ldc) {
+  __shared__ __align__(16) uint16_t ab[kFewHalves];  // [32 rows of A, 32 columns of Btp][k + 8]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int col = lane & 31, hh = lane >> 5;
+  const int k = n_kv * 128, stride = k + 8, c0 = 32 * blockIdx.y;
+  const int64_t row0 = (int64_t)blockIdx.x * 32;
+  uint16_t* bsm = ab + 32 * stride;
+  const uint16_t* bsrc = Btp + (int64_t)c0 * k;
+  const int per = k / 8;  // 16-byte pieces per column
+#pragma unroll 4
+  for (int p = tid & 15; p < per; p += 16) {  // per is a multiple of 16
+    uint4 v[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) v[j] = *(const uint4*)(bsrc + (int64_t)((tid >> 4) + 16 * j) * k + 8 * p);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) *(uint4*)(bsm + ((tid >> 4) + 16 * j) * stride + 8 * p) = v[j];
+  }
+  undo_rows<32, 256>(K, n_kv, seq, start, n_comp, m, phases, row0, ab);
+  __syncthreads();
+  if (tid >= 64) return;
+  float16v acc = {};
+  const uint16_t *ar = ab + col * stride + 8 * hh, *br = bsm + col * stride + 8 * hh;
+  for (int s0 = 0; s0 < k; s0 += 128)  // k is a multiple of 128
+#pragma unroll
+    for (int s = 0; s < 128; s += 16)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const half8*)(ar + s0 + s), *(const half8*)(br + s0 + s),
+                                                   acc, 0, 0, 0);
+  const float bz = bias ? bias[c0 + col] : 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int64_t rr = row0 + 8 * (e >> 2) + 4 * hh + (e & 3);
+    if (rr < m) C[rr * ldc + c0 + col] = acc[e] - bz;
+  }
+}
+
 // (cos, sin)(fl(pos * inv_freq[i])) for pos = start + t, t < n, i < hd2: the
 // phases of k_k_prepare, one table per token range (shared by every batch
 // row, head and layer that undoes RoPE at those positions).
@@ -531,6 +695,53 @@ extern "C" int shard_rope_phases(int32_t start, int32_t n, int32_t hd2, const fl
   return SHARD_OK;
 }
 
+// The kernel for few rows whose workgroups still fit one per CU and whose
+// operands fit LDS; false: none, k_pca_project_rope takes the call.  Measured
+// on MI355X at k = 1,024 and 192 columns, us (k_pca_project_rope: 30 up to
+// 4,096 rows, 38 at 16,384, 42 at 32,768):
+//   k_pca_rope_block    9.5 at 512 and 1,003 rows (192 workgroups); two rounds
+//                       and 19 or more past 256 workgroups
+//   k_pca_rope_rows<1>  18.8 at 1,003 rows, 19.2 at 4,096, 38.3 at 16,384
+//   k_pca_rope_rows<2>  24.1 at 4,096 rows, 27.1 at 16,384, 51.9 at 32,768
+static bool pca_rope_few(const uint16_t* K, int n_kv, int seq, int start, int n_comp, int64_t m,
+                         const float2* ph, const uint16_t* btp, int nb, const float* bias, float* c,
+                         int64_t ldc, hipStream_t s) {
+  constexpr int64_t kCUs = 256;
+  const int lds32 = 32 * (n_kv * 128 + 8);  // halves of 32 operand rows
+  const int64_t t32 = (m + 31) / 32, t64 = (m + 63) / 64;
+  auto go = [&](auto kern, int64_t tiles, int cols, int threads) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)cols), dim3(threads), 0, s, K, n_kv, seq,
+                       start, n_comp, m, ph, btp, bias, c, ldc);
+    return true;
+  };
+  if (t32 * nb <= kCUs && 2 * lds32 <= kFewHalves) return go(&k_pca_rope_block, t32, nb, 256);
+  if (t32 <= kCUs && lds32 <= kFewHalves) {
+    switch (nb) {
+      case 1: return go(&k_pca_rope_rows<1, 1>, t32, 1, 256);
+      case 2: return go(&k_pca_rope_rows<2, 1>, t32, 1, 256);
+      case 3: return go(&k_pca_rope_rows<3, 1>, t32, 1, 256);
+      case 4: return go(&k_pca_rope_rows<4, 1>, t32, 1, 256);
+      case 5: return go(&k_pca_rope_rows<5, 1>, t32, 1, 320);
+      case 6: return go(&k_pca_rope_rows<6, 1>, t32, 1, 384);
+      case 7: return go(&k_pca_rope_rows<7, 1>, t32, 1, 448);
+      default: return go(&k_pca_rope_rows<8, 1>, t32, 1, 512);
+    }
+  }
+  if (t64 <= kCUs && 2 * lds32 <= kFewHalves) {
+    switch (nb) {
+      case 1: return go(&k_pca_rope_rows<1, 2>, t64, 1, 256);
+      case 2: return go(&k_pca_rope_rows<2, 2>, t64, 1, 256);
+      case 3: return go(&k_pca_rope_rows<3, 2>, t64, 1, 256);
+      case 4: return go(&k_pca_rope_rows<4, 2>, t64, 1, 256);
+      case 5: return go(&k_pca_rope_rows<5, 2>, t64, 1, 320);
+      case 6: return go(&k_pca_rope_rows<6, 2>, t64, 1, 384);
+      case 7: return go(&k_pca_rope_rows<7, 2>, t64, 1, 448);
+      default: return go(&k_pca_rope_rows<8, 2>, t64, 1, 512);
+    }
+  }
+  return false;
+}
+
 extern "C" int shard_pca_project_rope(const uint16_t* k, int32_t batch, int32_t n_kv, int32_t seq,
                                       int32_t hd, int32_t start, int32_t n_comp,
                                       const float* phases, const uint16_t* btp, int32_t n,
@@ -545,6 +756,10 @@ extern "C" int shard_pca_project_rope(const uint16_t* k, int32_t batch, int32_t 
   const int64_t m = (int64_t)batch * n_comp;
   hipStream_t s = (hipStream_t)stream;
   dim3 grid((unsigned)((m + kPcaRows - 1) / kPcaRows));
+  if (pca_rope_few(k, n_kv, seq, start, n_comp, m, (const float2*)phases, btp, n / 32, bias, c, ldc, s)) {
+    SHARD_LAUNCH_CHECK("shard_pca_project_rope");
+    return SHARD_OK;
+  }
 #define SHARD_PR(NB) hipLaunchKernelGGL(k_pca_project_rope<NB>, grid, dim3(kPcaThreads), 0, s, k, n_kv, \
                                         seq, start, n_comp, m, (const float2*)phases, btp, bias, c, ldc)
   switch (n / 32) {

@@ -833,3 +833,29 @@ def test_rope_stream_append_dev_row(cuda, qjl):
         assert torch.equal(q_got, q_want), row
         for n in order + (qorder if qjl else ()):
             assert torch.equal(got[n], want[n]), (row, n)
+
+
+@pytest.mark.parametrize("B,G,T,n,start,n_comp", [
+    (1, 8, 40, 192, 0, 40), (3, 8, 70, 192, 5, 33), (1, 1, 9, 32, 1, 5), (2, 4, 2100, 64, 4, 2033),
+    (1, 8, 2049, 256, 0, 2049), (1, 16, 300, 96, 2, 290), (4, 8, 2100, 128, 0, 2100),
+    (5, 8, 8200, 160, 3, 3300), (1, 20, 100, 32, 0, 100)])
+def test_pca_project_rope_few_rows(cuda, B, G, T, n, start, n_comp):
+    """The projection's kernels for few rows (a block of C per workgroup, 32
+    and 64 rows per workgroup, and the 128-row kernel past them and past 19 kv
+    heads) at ragged row counts, several batch rows per tile and every column
+    count: the fp32 sums of the fp16 operand k_prepare writes, and rows past m
+    untouched."""
+    from shard_amd import bench_data, ops
+    g = torch.Generator().manual_seed(n_comp)
+    k = torch.randn(B, G, T, 128, generator=g).half().to(cuda)
+    bt = (torch.randn(n, G * 128, generator=g) / 32).half().to(cuda)
+    inv = bench_data.inv_freq().to(cuda)
+    bias = torch.randn(n, generator=g).to(cuda)
+    ph = ops.rope_phases(start, n_comp, inv)
+    got = ops.pca_project_rope(k, start, n_comp, ph, ops.rope_basis(bt), bias)
+    a = ops.k_prepare(k, start, n_comp, inv, torch.zeros(G * 128, device=cuda))
+    want = a.double() @ bt.double().t().contiguous() - bias.double()
+    # fp32 sums of G * 128 products: about sqrt(k) ulps of their magnitude
+    tol = 1e-6 * (G * 128) ** 0.5 * float((a.double().abs() @ bt.double().abs().t().contiguous()).max())
+    assert got.shape == (B * n_comp, n)
+    assert float((got.double() - want).abs().max()) <= tol
