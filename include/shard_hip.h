@@ -420,6 +420,11 @@ int shard_decode_prepare(const uint16_t* k_basis, const uint16_t* k_coeff_scale,
                          int32_t head_dim, int32_t rank, void* out, size_t out_bytes,
                          void* stream);
 
+/* A boolean attention mask (n bytes, nonzero = attend) as the additive fp32
+ * mask shard_decode_attn reads: 0 where set, the lowest fp32 value elsewhere
+ * (what transformers' own float masks hold). */
+int shard_mask_additive(const uint8_t* mask, int64_t n, float* out, void* stream);
+
 /* 1 when shard_decode_attn takes the shapes in `args` (head_dim 128 with up
  * to 64 query heads per kv head, or head_dim 64 with an even number of kv
  * heads and up to 32 query heads per kv head; rank a multiple of 32 up to 256;

@@ -1763,6 +1763,14 @@ int decode_attn_tok(const shard_decode_args* a, float* ws, hipStream_t s) {
   return launch_merge(a, ws, pl.ns, s);
 }
 
+// A boolean attention mask (nonzero = attend) as the additive fp32 mask the
+// decode kernels read: 0, or the lowest fp32 value.
+__global__ void k_mask_additive(const uint8_t* __restrict__ mask, int64_t n, float* __restrict__ out) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    out[i] = mask[i] ? 0.f : -3.402823466e+38f;
+}
+
 }  // namespace shard
 
 using namespace shard;
@@ -1797,6 +1805,14 @@ int shard_decode_prepare(const uint16_t* k_basis, const uint16_t* k_coeff_scale,
   hipLaunchKernelGGL(k_decode_prepare, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
                      k_basis, k_coeff_scale, k_mean, inv_freq, G, rank, hp, op, rope);
   SHARD_LAUNCH_CHECK("shard_decode_prepare");
+  return SHARD_OK;
+}
+
+int shard_mask_additive(const uint8_t* mask, int64_t n, float* out, void* stream) {
+  if (!mask || !out || n <= 0) return SHARD_ERR_ARG;
+  hipLaunchKernelGGL(k_mask_additive, dim3((unsigned)grid_cap((n + 255) / 256, 4096)), dim3(256), 0,
+                     (hipStream_t)stream, mask, n, out);
+  SHARD_LAUNCH_CHECK("shard_mask_additive");
   return SHARD_OK;
 }
 

@@ -859,3 +859,14 @@ def test_pca_project_rope_few_rows(cuda, B, G, T, n, start, n_comp):
     tol = 1e-6 * (G * 128) ** 0.5 * float((a.double().abs() @ bt.double().abs().t().contiguous()).max())
     assert got.shape == (B * n_comp, n)
     assert float((got.double() - want).abs().max()) <= tol
+
+
+@pytest.mark.parametrize("n", [1, 63, 256, 100003])
+def test_mask_additive_equals_torch(cuda, n):
+    """A boolean mask on the GPU becomes 0 / the fp32 minimum in one launch, as
+    the torch expression for other devices and layouts."""
+    from shard_amd.ops import additive_mask
+    m = torch.rand(2, n, generator=torch.Generator().manual_seed(n)) < 0.5
+    want = additive_mask(m)
+    assert torch.equal(additive_mask(m.to(cuda)).cpu(), want)
+    assert torch.equal(additive_mask(m.to(cuda).t()).cpu(), want.t())
