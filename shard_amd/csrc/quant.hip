@@ -1252,15 +1252,45 @@ __global__ __launch_bounds__(256) void k_vq_assign_table(
 // Deterministic k-means update: stable counting sort of the rows by centroid
 // into a sorted copy, then each (centroid, dim) sums its rows in increasing
 // row order (torch CPU index_add_ order), divides by the count, and keeps
-// empty centroids.
-//   blk[q * nblk + b]: rows of block b (KM_R rows) with centroid q; after the
-//   scan, the first slot of those rows within centroid q's run.
+// empty centroids.  A large set is sorted in segments of consecutive rows: one
+// launch sorts segment i and adds segment i - 1 to the running sums.
+//   blk[q * nblk + b]: rows of block b (km_rows rows) with centroid q; after
+//   the scan, the first slot of those rows within centroid q's run of its
+//   segment.
 // ---------------------------------------------------------------------------
-constexpr int KM_R = 4096;   // rows per block of the counting sort
+// Rows per block of the counting sort: 4,096 where that gives 2,048 blocks or
+// more, else as few as 256 (a block is one wave of the scatter; 124 blocks at
+// a 2K-token layer's 507K rows left it waiting on latency, 42 us against 11;
+// the whole update 90 us, now 52).
+inline int km_rows(int64_t n) {
+  const int64_t r = (n / 2048 + 255) & ~(int64_t)255;
+  return (int)(r < 256 ? 256 : r > 4096 ? 4096 : r);
+}
+// Segments of the sort, of 500K rows or more: the sums are chains of dependent
+// adds (about 8 clocks a row of the largest centroid, 1.75 ms at 67M rows) on
+// a few lanes per CU, the scatter (1.18 ms there) fills the others meanwhile.
+// One update at 67M rows: 3.37 ms with the two in turn, 2.92 in 8 segments,
+// 2.74 in 16 (chunks of 512 rows instead of 1,024 in the sums: 3.08); at 8.4M
+// 0.49 and 0.39.
+constexpr int kKmMaxSegs = 16;
+struct KmPlan {
+  int R, segs;
+  int64_t nblk, bps;  // blocks, blocks per segment
+};
+inline KmPlan km_plan(int64_t n) {
+  KmPlan p;
+  p.R = km_rows(n);
+  p.nblk = (n + p.R - 1) / p.R;
+  const int64_t want = n / 500000;
+  p.segs = (int)(want < 2 ? 1 : want > kKmMaxSegs ? kKmMaxSegs : want);
+  p.bps = (p.nblk + p.segs - 1) / p.segs;
+  p.segs = (int)((p.nblk + p.bps - 1) / p.bps);
+  return p;
+}
 constexpr int KM_DMAX = 8;   // widest rows the sorted copy holds
 
 __global__ __launch_bounds__(256) void k_km_hist(const int32_t* __restrict__ idx, int64_t n, int k,
-                                                 int64_t nblk, int32_t* __restrict__ blk) {
+                                                 int KM_R, int64_t nblk, int32_t* __restrict__ blk) {
   __shared__ int32_t h[1024];
   for (int i = threadIdx.x; i < k; i += blockDim.x) h[i] = 0;
   __syncthreads();
@@ -1271,18 +1301,19 @@ __global__ __launch_bounds__(256) void k_km_hist(const int32_t* __restrict__ idx
   for (int q = threadIdx.x; q < k; q += blockDim.x) blk[(int64_t)q * nblk + blockIdx.x] = h[q];
 }
 
-// For each centroid (one workgroup): exclusive scan of its per-block counts
-// (contiguous, 256 at a time: wave scans, then the four wave totals) in place,
-// and its total count.
+// For each centroid and segment (one workgroup): exclusive scan of its
+// per-block counts (contiguous, 256 at a time: wave scans, then the four wave
+// totals) in place, and its total count in the segment.
 __global__ __launch_bounds__(256) void k_km_scan_blocks(int32_t* __restrict__ blk, int64_t nblk,
-                                                        int32_t* __restrict__ count) {
+                                                        int64_t bps, int32_t* __restrict__ count) {
   __shared__ int32_t wsum[4];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   int32_t* row = blk + (int64_t)blockIdx.x * nblk;
+  const int64_t b0 = (int64_t)blockIdx.y * bps, b1 = b0 + bps < nblk ? b0 + bps : nblk;
   int32_t carry = 0;
-  for (int64_t base = 0; base < nblk; base += 256) {
+  for (int64_t base = b0; base < b1; base += 256) {
     const int64_t i = base + t;
-    const int32_t v = i < nblk ? row[i] : 0;
+    const int32_t v = i < b1 ? row[i] : 0;
     int32_t sc = v;  // inclusive scan over the wave
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -1293,55 +1324,78 @@ __global__ __launch_bounds__(256) void k_km_scan_blocks(int32_t* __restrict__ bl
     __syncthreads();
     int32_t pre = carry;
     for (int u = 0; u < w; ++u) pre += wsum[u];
-    if (i < nblk) row[i] = pre + sc - v;
+    if (i < b1) row[i] = pre + sc - v;
     carry += wsum[0] + wsum[1] + wsum[2] + wsum[3];
     __syncthreads();  // wsum is rewritten by the next round
   }
-  if (t == 0) count[blockIdx.x] = carry;
+  if (t == 0) count[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = carry;
 }
 
-__global__ void k_km_offsets(const int32_t* __restrict__ count, int k, int32_t* __restrict__ off) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    int32_t run = 0;
-    for (int q = 0; q < k; ++q) {
-      off[q] = run;
-      run += count[q];
-    }
+// Per segment (one workgroup, thread = centroid, k <= 1024): the first slot of
+// each centroid's run, the segment's rows keeping their place in the copy; and
+// the cleared maximum step.
+__global__ __launch_bounds__(1024) void k_km_offsets(const int32_t* __restrict__ count, int k,
+                                                     int64_t seg_rows, int32_t* __restrict__ off,
+                                                     uint32_t* __restrict__ maxd) {
+  __shared__ int32_t wsum[16];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int64_t at = (int64_t)blockIdx.x * k + t;
+  const int32_t v = t < k ? count[at] : 0;
+  int32_t sc = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int32_t u = __shfl_up(sc, o, 64);
+    if (lane >= o) sc += u;
   }
+  if (lane == 63) wsum[w] = sc;
+  __syncthreads();
+  for (int u = 0; u < w; ++u) sc += wsum[u];
+  if (t < k) off[at] = (int32_t)(blockIdx.x * seg_rows) + sc - v;
+  if (t == 0 && blockIdx.x == 0) *maxd = 0u;
 }
 
-// One wave per block of KM_R rows, 64 rows per round in increasing order.  A
+struct KmArgs {
+  const float* x;
+  const int32_t* idx;
+  int64_t n, nblk;
+  int32_t k, R;
+  const int32_t *blk, *count, *off;  // count, off: (segment, centroid)
+  float *xs, *acc;                   // sorted copy; running sums (k, D)
+  const float* c;
+  float* newc;
+  uint32_t* maxd;
+  int32_t segs;
+  // this launch: sort blocks [b0, b1) (segment `sort`), and add segment `sum`
+  int64_t b0, b1;
+  int32_t sort, sum;  // -1: none
+};
+
+// One wave per block of R rows, 64 rows per round in increasing order.  A
 // row's slot is its centroid's running count in the block (LDS) plus the
 // number of lower lanes of the round with the same centroid (lanes that agree
 // on every bit of the centroid index, from one ballot per bit); the last lane
 // of each centroid's group then advances the count.  The row's D values go to
 // the sorted copy at that slot.
 template <int D>
-__global__ __launch_bounds__(64) void k_km_scatter(const float* __restrict__ x,
-                                                   const int32_t* __restrict__ idx, int64_t n,
-                                                   int k, int64_t nblk,
-                                                   const int32_t* __restrict__ blk,
-                                                   const int32_t* __restrict__ off,
-                                                   float* __restrict__ xs) {
-  __shared__ int32_t run[1024];
-  const int lane = threadIdx.x;
-  const int64_t b = blockIdx.x;
-  for (int q = lane; q < k; q += 64) run[q] = off[q] + blk[(int64_t)q * nblk + b];
-  __syncthreads();
+__device__ __forceinline__ void km_scatter(const KmArgs& a, const int64_t b, int32_t* run) {
+  const int lane = threadIdx.x & 63, k = a.k;
+  for (int q = lane; q < k; q += 64)
+    run[q] = a.off[(int64_t)a.sort * k + q] + a.blk[(int64_t)q * a.nblk + b];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   const int nbits = k > 1 ? 32 - __builtin_clz((unsigned)(k - 1)) : 0;
   const uint64_t below = (1ull << lane) - 1ull;
-  const int64_t r0 = b * KM_R;
+  const int64_t r0 = b * a.R;
   constexpr int RU = 4;  // rounds whose loads go out together
-  for (int rr = 0; rr < KM_R && r0 + rr < n; rr += 64 * RU) {
+  for (int rr = 0; rr < a.R && r0 + rr < a.n; rr += 64 * RU) {
     int key[RU];
     float xv[RU][D];
 #pragma unroll
     for (int u = 0; u < RU; ++u) {
       const int64_t r = r0 + rr + 64 * u + lane;
-      const bool valid = rr + 64 * u < KM_R && r < n;
-      key[u] = valid ? idx[r] : -1;
+      const bool valid = rr + 64 * u < a.R && r < a.n;
+      key[u] = valid ? a.idx[r] : -1;
 #pragma unroll
-      for (int j = 0; j < D; ++j) xv[u][j] = valid ? x[r * D + j] : 0.f;
+      for (int j = 0; j < D; ++j) xv[u][j] = valid ? a.x[r * D + j] : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < RU; ++u) {
@@ -1361,32 +1415,31 @@ __global__ __launch_bounds__(64) void k_km_scatter(const float* __restrict__ x,
       if (valid && rank == grp - 1) run[kk] += grp;
       if (valid) {
 #pragma unroll
-        for (int j = 0; j < D; ++j) xs[(int64_t)slot * D + j] = xv[u][j];
+        for (int j = 0; j < D; ++j) a.xs[(int64_t)slot * D + j] = xv[u][j];
       }
     }
   }
 }
 
-// One workgroup per centroid over its run of the sorted copy (increasing row
-// order).  Chunks of 256 P rows are loaded (coalesced) one chunk ahead and
-// staged in LDS dim-major (columns padded so the D lanes read distinct
-// banks), double-buffered; lanes 0..D-1 of wave 0 add them in order, one
-// running sum per dim, with the LDS reads of the next 32 values in flight
-// while the current 32 are added.
+// One workgroup per centroid over its run of a segment (increasing row order).
+// Chunks of 256 P rows are loaded (coalesced) one chunk ahead and staged in
+// LDS dim-major (columns padded so the D lanes read distinct banks),
+// double-buffered; lanes 0..D-1 of wave 0 add them in order to the running sum
+// of the segments before, one per dim, with the LDS reads of the next 32
+// values in flight while the current 32 are added.
 template <int D>
-__global__ __launch_bounds__(256) void k_km_sum(const float* __restrict__ xs,
-                                                const int32_t* __restrict__ count,
-                                                const int32_t* __restrict__ off,
-                                                const float* __restrict__ c, int k,
-                                                float* __restrict__ newc, uint32_t* __restrict__ maxd) {
-  constexpr int P = D <= 4 ? 4 : 2;  // rows per thread per chunk
-  constexpr int CH = 256 * P;        // rows per chunk
-  constexpr int CS = CH + 4;         // column stride
-  __shared__ __align__(16) float buf[2][D][CS];
-  const int q = blockIdx.x;
+struct KmSum {
+  static constexpr int P = D <= 4 ? 4 : 2;  // rows per thread per chunk
+  static constexpr int CH = 256 * P; // rows per chunk
+  static constexpr int CS = CH + 4;  // column stride
+  float buf[2][D][CS];
+};
+template <int D>
+__device__ __forceinline__ void km_sum(const KmArgs& a, const int q, KmSum<D>& L) {
+  constexpr int P = KmSum<D>::P, CH = KmSum<D>::CH;
   const int t = threadIdx.x;
-  const int32_t cnt = count[q];
-  const float* src = xs + (int64_t)off[q] * D;
+  const int32_t cnt = a.count[(int64_t)a.sum * a.k + q];
+  const float* src = a.xs + (int64_t)a.off[(int64_t)a.sum * a.k + q] * D;
   float xv[P][D];
   auto load = [&](int32_t base) {
 #pragma unroll
@@ -1399,21 +1452,21 @@ __global__ __launch_bounds__(256) void k_km_sum(const float* __restrict__ xs,
     }
   };
   load(0);
-  float acc = 0.f;
+  float acc = a.sum > 0 && t < D ? a.acc[q * D + t] : 0.f;
   int cur = 0;
   for (int32_t base = 0; base < cnt; base += CH) {
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       if (base + 256 * p + t < cnt) {
 #pragma unroll
-        for (int j = 0; j < D; ++j) buf[cur][j][256 * p + t] = xv[p][j];
+        for (int j = 0; j < D; ++j) L.buf[cur][j][256 * p + t] = xv[p][j];
       }
     }
     __syncthreads();
     load(base + CH);
     if (t < D) {
       const int n_here = cnt - base < CH ? cnt - base : CH;
-      const float* col = buf[cur][t];
+      const float* col = L.buf[cur][t];
       const float4* c4 = (const float4*)col;
       const int nb = n_here >> 5;  // blocks of 32 values
       float4 va[8], vb[8];
@@ -1446,14 +1499,47 @@ __global__ __launch_bounds__(256) void k_km_sum(const float* __restrict__ xs,
   }
   if (t < D) {
     const int idx = q * D + t;
-    const float old = c[idx];
-    const float nv = cnt > 0 ? div_rn(acc, (float)cnt) : old;
-    newc[idx] = nv;
-    atomicMax(maxd, __float_as_uint(fabsf(sub_rn(nv, old))));
+    if (a.sum < a.segs - 1) {
+      a.acc[idx] = acc;
+      return;
+    }
+    int32_t total = 0;
+    for (int s = 0; s < a.segs; ++s) total += a.count[(int64_t)s * a.k + q];
+    const float old = a.c[idx];
+    const float nv = total > 0 ? div_rn(acc, (float)total) : old;
+    a.newc[idx] = nv;
+    atomicMax(a.maxd, __float_as_uint(fabsf(sub_rn(nv, old))));
   }
 }
 
-__global__ void k_km_zero(uint32_t* p) { *p = 0u; }
+// Workgroups [0, k) add segment a.sum (dispatched first, their adding wave at
+// a higher priority); the others sort blocks a.b0 .. a.b1, one per wave.
+template <int D>
+__global__ __launch_bounds__(256) void k_km_step(const KmArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int n_sum = a.sum >= 0 ? a.k : 0;
+  if ((int)blockIdx.x < n_sum) {
+    if (threadIdx.x < 64) __builtin_amdgcn_s_setprio(3);
+    km_sum<D>(a, (int)blockIdx.x, *(KmSum<D>*)smem);
+    return;
+  }
+  const int w = threadIdx.x >> 6;
+  const int64_t b = a.b0 + ((int64_t)blockIdx.x - n_sum) * 4 + w;
+  if (b < a.b1) km_scatter<D>(a, b, (int32_t*)smem + (int64_t)w * a.k);
+}
+
+template <int D>
+void km_steps(KmArgs a, const KmPlan& pl, hipStream_t s) {
+  for (int i = 0; i <= pl.segs; ++i) {
+    a.sort = i < pl.segs ? i : -1;
+    a.sum = i - 1;
+    a.b0 = i * pl.bps;
+    a.b1 = a.sort < 0 ? a.b0 : std::min(a.b0 + pl.bps, pl.nblk);
+    const int64_t wgs = (a.b1 - a.b0 + 3) / 4 + (a.sum >= 0 ? a.k : 0);
+    const size_t lds = std::max(a.sum >= 0 ? sizeof(KmSum<D>) : 0, a.sort >= 0 ? (size_t)16 * a.k : 0);
+    hipLaunchKernelGGL(k_km_step<D>, dim3((unsigned)wgs), dim3(256), lds, s, a);
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Per-token 8-bit Lloyd-Max stream quantizer (cache.py:207-215, streaming.py:59-72)
@@ -2112,12 +2198,16 @@ int shard_vq_assign_table(const float* x, int64_t n, const float* centroids, int
   return SHARD_OK;
 }
 
+static int64_t km_ints(const KmPlan& p, int32_t k, int32_t d) {
+  return (p.nblk * k + 2 * (int64_t)k * p.segs + (int64_t)k * d + 3) & ~(int64_t)3;
+}
+
 size_t shard_kmeans_update_workspace_d(int64_t n, int32_t k, int32_t d) {
   if (n <= 0 || k <= 0 || d <= 0 || d > KM_DMAX) return 0;
-  const int64_t nblk = (n + KM_R - 1) / KM_R;
-  // per-block counts, counts, offsets, then the sorted copy of the rows
-  const int64_t ints = ((nblk * k + 2 * (int64_t)k) + 3) & ~(int64_t)3;
-  return (size_t)ints * sizeof(int32_t) + (size_t)n * d * sizeof(float);
+  const KmPlan p = km_plan(n);
+  // per-block counts, counts and offsets per segment, running sums, then the
+  // sorted copy of the rows
+  return (size_t)km_ints(p, k, d) * sizeof(int32_t) + (size_t)n * d * sizeof(float);
 }
 
 size_t shard_kmeans_update_workspace(int64_t n, int32_t k) {
@@ -2134,33 +2224,26 @@ int shard_kmeans_update(const float* x, int64_t n, int32_t d, const int32_t* idx
   if (n > INT32_MAX) return SHARD_ERR_SHAPE;  // slots are int32
   if (!workspace || workspace_bytes < shard_kmeans_update_workspace_d(n, k, d)) return SHARD_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
-  const int64_t nblk = (n + KM_R - 1) / KM_R;
+  const KmPlan pl = km_plan(n);
   int32_t* blk = (int32_t*)workspace;
-  int32_t* count = blk + nblk * k;
-  int32_t* off = count + k;
-  float* xs = (float*)(blk + (((nblk * k + 2 * (int64_t)k) + 3) & ~(int64_t)3));
-  hipLaunchKernelGGL(k_km_hist, dim3((unsigned)nblk), dim3(256), 0, s, idx, n, k, nblk, blk);
-  hipLaunchKernelGGL(k_km_scan_blocks, dim3((unsigned)k), dim3(256), 0, s, blk, nblk, count);
-  hipLaunchKernelGGL(k_km_offsets, dim3(1), dim3(64), 0, s, count, k, off);
-  hipLaunchKernelGGL(k_km_zero, dim3(1), dim3(1), 0, s, (uint32_t*)max_delta);
-  const unsigned kb = (unsigned)k, nb = (unsigned)nblk;
+  int32_t* count = blk + pl.nblk * k;
+  int32_t* off = count + (int64_t)k * pl.segs;
+  KmArgs a = {};
+  a.x = x; a.idx = idx; a.n = n; a.nblk = pl.nblk; a.k = k; a.R = pl.R;
+  a.blk = blk; a.count = count; a.off = off;
+  a.acc = (float*)(off + (int64_t)k * pl.segs);
+  a.xs = (float*)(blk + km_ints(pl, k, d));
+  a.c = centroids; a.newc = new_centroids; a.maxd = (uint32_t*)max_delta; a.segs = pl.segs;
+  hipLaunchKernelGGL(k_km_hist, dim3((unsigned)pl.nblk), dim3(256), 0, s, idx, n, k, pl.R, pl.nblk, blk);
+  hipLaunchKernelGGL(k_km_scan_blocks, dim3((unsigned)k, (unsigned)pl.segs), dim3(256), 0, s, blk, pl.nblk,
+                     pl.bps, count);
+  hipLaunchKernelGGL(k_km_offsets, dim3((unsigned)pl.segs), dim3(1024), 0, s, count, k, pl.bps * pl.R, off,
+                     a.maxd);
   switch (d) {
-    case 1:
-      hipLaunchKernelGGL(k_km_scatter<1>, dim3(nb), dim3(64), 0, s, x, idx, n, k, nblk, blk, off, xs);
-      hipLaunchKernelGGL(k_km_sum<1>, dim3(kb), dim3(256), 0, s, xs, count, off, centroids, k, new_centroids, (uint32_t*)max_delta);
-      break;
-    case 2:
-      hipLaunchKernelGGL(k_km_scatter<2>, dim3(nb), dim3(64), 0, s, x, idx, n, k, nblk, blk, off, xs);
-      hipLaunchKernelGGL(k_km_sum<2>, dim3(kb), dim3(256), 0, s, xs, count, off, centroids, k, new_centroids, (uint32_t*)max_delta);
-      break;
-    case 4:
-      hipLaunchKernelGGL(k_km_scatter<4>, dim3(nb), dim3(64), 0, s, x, idx, n, k, nblk, blk, off, xs);
-      hipLaunchKernelGGL(k_km_sum<4>, dim3(kb), dim3(256), 0, s, xs, count, off, centroids, k, new_centroids, (uint32_t*)max_delta);
-      break;
-    default:
-      hipLaunchKernelGGL(k_km_scatter<8>, dim3(nb), dim3(64), 0, s, x, idx, n, k, nblk, blk, off, xs);
-      hipLaunchKernelGGL(k_km_sum<8>, dim3(kb), dim3(256), 0, s, xs, count, off, centroids, k, new_centroids, (uint32_t*)max_delta);
-      break;
+    case 1: km_steps<1>(a, pl, s); break;
+    case 2: km_steps<2>(a, pl, s); break;
+    case 4: km_steps<4>(a, pl, s); break;
+    default: km_steps<8>(a, pl, s); break;
   }
   SHARD_LAUNCH_CHECK("shard_kmeans_update");
   return SHARD_OK;

@@ -472,20 +472,27 @@ def kmeans(data: torch.Tensor, k: int, n_iter: int = 30, seed: int = 42):
     tab_ws = None
     if n >= VQ_TABLE_MIN_ROWS and VqTable.supported(centroids):
         tab_ws = _workspace(lib.shard_vq_assign_table_workspace(n), data.device)
-    idx = None
-    deltas = []
+    idx = last = None
     for it in range(n_iter):
         if tab_ws is not None:
             idx = vq_assign_table(data, VqTable(centroids), tab_ws)
         else:
             idx = vq_assign(data, centroids)
-        new, maxd = kmeans_update(data, idx, centroids, ws)
-        deltas.append(maxd)
-        # one host sync per iteration, as the reference's .item() (cache.py:36)
-        if it >= 5 and maxd.item() < 1e-4:
-            centroids = new
-            break
-        centroids = new
+        centroids, maxd = kmeans_update(data, idx, centroids, ws)
+        # the reference reads max |delta| here (cache.py:36); it is read one
+        # iteration later instead, while the GPU works on the next one, which
+        # is dropped when the step was the last
+        step = None
+        if it >= 5:
+            host_max = torch.empty(1, dtype=torch.float32, pin_memory=True)
+            host_max.copy_(maxd, non_blocking=True)
+            step = (centroids, idx, host_max, torch.cuda.Event())
+            step[3].record(torch.cuda.current_stream(data.device))
+        if last is not None:
+            last[3].synchronize()
+            if last[2].item() < 1e-4:
+                return last[0], last[1]
+        last = step
     return centroids, idx
 
 

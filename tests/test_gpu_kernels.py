@@ -501,6 +501,27 @@ def test_kmeans_update_bitexact(cuda, n, k, d, assign):
     assert maxd.item() == (new - c).abs().max().item()
 
 
+@pytest.mark.parametrize("n,k,d", [(999999, 7, 4), (1000003, 7, 1), (1600000, 300, 2), (2100001, 256, 4),
+                                   (1100000, 1024, 8)])
+def test_kmeans_update_in_segments_bitexact(cuda, n, k, d):
+    """Sets sorted in one, two and four segments, each added to the running
+    sums while the next is sorted: the sequential sums of torch CPU index_add_,
+    a centroid without rows in the first segment or in any included."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(n, d, generator=g)
+    idx = torch.randint(0, k - 1, (n,), generator=g)
+    idx[: n // 2][idx[: n // 2] == 3] = 4
+    c = torch.randn(k, d, generator=g)
+    want, cnt = torch.zeros(k, d), torch.zeros(k)
+    want.index_add_(0, idx, x)
+    cnt.index_add_(0, idx, torch.ones(n))
+    want = torch.where(cnt[:, None] > 0, want / cnt[:, None], c)
+    got, maxd = ops.kmeans_update(x.to(cuda), idx.to(torch.int32).to(cuda), c.to(cuda))
+    assert np.array_equal(got.cpu().numpy(), want.numpy())
+    assert maxd.item() == (want - c).abs().max().item()
+
+
 def test_kmeans_matches_reference_golden(cuda, golden):
     ops = _ops()
     gld = golden("kmeans.npz")
