@@ -37,7 +37,8 @@ struct RebuildOut {
 // per token and head.  8,124 tokens x 8 heads of 128 dims, rank 192: the
 // scalar kernel's dot products from LDS took 242 us; a whole layer with V and
 // the segments (one torch.cat pass over each of K and V before) went from 290
-// to 28 us, batch 4 x 2,933 x 8 heads of 64 from 202 to 23 us.
+// to 27 us, batch 4 x 2,933 x 8 heads of 64 from 202 to 22.8 us.  Not kept: the
+// basis rows turned into operand order through LDS (30.2 us).
 template <int HD, int KS>
 struct RebuildLds {
   static constexpr int kRow = 16 * KS + 8;     // halves per coefficient row: 16 bytes of padding
@@ -307,7 +308,7 @@ __device__ __forceinline__ void rebuild_copy(const RebuildSegs& sg, const Rebuil
 // for the wide accesses (otherwise element by element).  Bound by the 256 bytes written per
 // row; one wave per row with a 2-byte store per lane took 18.7 us at
 // 8,124 x 8 rows of 128.
-constexpr int kRvSteps = 4;  // row groups per wave
+constexpr int kRvSteps = 1;  // row groups per wave: a whole 8K layer 27.0 us, with 4 29.3, with 8 31.7
 template <int HD, int LG>
 __global__ __launch_bounds__(256)
 void k_rebuild_v(const uint8_t* __restrict__ vidx, const uint16_t* __restrict__ vcb,
