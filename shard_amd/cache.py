@@ -623,14 +623,15 @@ class _EigJob:
     at p = 1024, most of it the 1,023 launches of the tridiagonalization, which
     a background thread issues; LAPACK on the host took 50 to 200 ms), checked
     for orthogonality and residual.  A layer that misses the bounds (clustered
-    or zero eigenvalues, a non-finite covariance) or is larger than the kernel
-    takes goes to the host's float64 eigh, errors included."""
+    or zero eigenvalues, a non-finite covariance), is larger than the kernel
+    takes or is asked for more pairs than it has (it gives them all) goes to
+    the host's float64 eigh, errors included."""
 
     def __init__(self, cov: torch.Tensor, rank: int):
         self.cov, self.rank = cov.detach(), rank
         self.future = None
         p = cov.shape[0]
-        if not cov.is_cuda or not 2 <= p <= ops.EIGH_MAX or rank < 1:
+        if not cov.is_cuda or not 2 <= p <= ops.EIGH_MAX or not 1 <= rank <= p:
             return
         self.main = torch.cuda.current_stream(cov.device)
         self.side = torch.cuda.Stream(cov.device)

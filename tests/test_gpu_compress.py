@@ -348,3 +348,12 @@ def test_eig_job_hands_clusters_and_bad_input_to_the_host(cuda):
         want, eig_want = _eigh_top(c.double(), 20)
         assert torch.equal(basis.cpu().nan_to_num(7.0), want.nan_to_num(7.0))
         assert torch.equal(eig.cpu().nan_to_num(7.0), eig_want.nan_to_num(7.0))
+
+
+def test_pca_basis_cov_of_fewer_columns_than_asked(cuda):
+    """More eigenpairs than the covariance has gives them all, on either device."""
+    from shard_amd.cache import pca_basis_cov
+    c = torch.diag(torch.arange(8.0, 0.0, -1.0))
+    for cov in (c, c.to(cuda)):
+        basis, eig = pca_basis_cov(cov, 20)
+        assert basis.shape == (8, 8) and torch.equal(eig.cpu(), torch.arange(8.0, 0.0, -1.0))
