@@ -1945,7 +1945,17 @@ int shard_decode_attn(const shard_decode_args* a, void* workspace, size_t worksp
 int shard_decode_attn_noalloc(const shard_decode_args* a, void* stream) {
   const int st = decode_attn_check(a);
   if (st != SHARD_OK) return st;
-  const size_t need = shard_decode_attn_workspace(a);
+  size_t need = shard_decode_attn_workspace(a);
+  shard_decode_args tok;
+  if (need > SHARD_DECODE_NOALLOC_SCRATCH_BYTES && a->kernel == 0) {
+    // a large batch with many extra tokens: the row-split kernel writes a
+    // partial row per 128 of them and head, the token-tiled one at most about
+    // one per CU and query head of its group
+    tok = *a;
+    tok.kernel = 2;
+    a = &tok;
+    need = shard_decode_attn_workspace(a);
+  }
   if (need > SHARD_DECODE_NOALLOC_SCRATCH_BYTES) {
     char msg[160];
     snprintf(msg, sizeof(msg),
