@@ -271,7 +271,7 @@ void k_tri_eig(const double* __restrict__ dg, const double* __restrict__ eg, int
 
 // Row m of Z (an eigenvector of the tridiagonal matrix) times the reflectors,
 // last column's first: z -= tau_k (v_k . z) v_k.  One wave per vector, the
-// vector in registers, the next reflectors' loads in flight (4 deep).
+// vector in registers, the next reflector's loads in flight.
 __global__ __launch_bounds__(64)
 void k_back(const double* __restrict__ V, const double* __restrict__ tau, int n,
             double* __restrict__ Z) {
