@@ -9,7 +9,7 @@
 //     tile: wave P rebuilds rows of the 16 RoPE pairs [16 P, 16 P + 16) (basis
 //     operand in VGPRs), the partial scores meet in LDS, then a shared online
 //     softmax and VQ value sum.  The extra tokens (at most 2048) run on
-//     workgroups of their own, 128 tokens each, one more partial row per
+//     workgroups of their own, 128 tokens a pass, one more partial row per
 //     query head and workgroup.
 //   k_decode_tok (token-tiled)  grid = n_splits * n_kv * query groups * B,
 //     512-thread workgroups, one per CU, 1, 2 or 4 query heads per workgroup;
@@ -376,13 +376,18 @@ static_assert(kTG == 1 || kTG == 2, "SHARD_DECODE_TG must be 1 or 2");
 // layer-step against 13.3.  Within the rule the two are close (1.5K: 14.8 us
 // against 15.0 with 78 extra tokens, 15.1 against 14.7 with 132).
 constexpr int kXFew = 256, kXShort = 16, kXLong = 32;
+// A pass of an extra-token workgroup in compressed tiles of its neighbours: it
+// takes 3.0 us, a tile of two workgroups per CU 1.15 (4 x 2,200 tokens with
+// 1,968 extra, 2 to 16 passes: 11.5 us + 3.0 a pass).
+constexpr int kXPassTiles = 3;
 
-// Extra tokens (sink, window, decode, stream; fp16 rows) xi XT .. xi XT + XT of
-// kv head g, XT = NW x_wave, on a workgroup of their own: scores on MFMA (rows =
-// the kGQA query heads, k = head dims, columns = the wave's 32 tokens),
-// softmax per head (wave h < kGQA owns head h), values accumulated
-// lane-per-dim pair.  Writes partial row `split` of each query head, in the
-// plain (not rotated) basis; empty (m = -inf) when the call has fewer tokens.
+// Extra tokens (sink, window, decode, stream; fp16 rows) of kv head g on
+// workgroups of their own: workgroup xi takes passes xi, xi + n_xs, ... of XT =
+// NW x_wave tokens each.  Scores on MFMA (rows = the kGQA query heads, k = head
+// dims, columns = the wave's 32 tokens), online softmax per head (wave h < kGQA
+// owns head h), values accumulated lane-per-dim pair.  Writes partial row
+// `split` of each query head, in the plain (not rotated) basis; empty (m =
+// -inf) when the call has fewer tokens.
 // A pass takes about 14K clocks whatever it holds, the time of several
 // compressed tiles: run by one workgroup before its tiles, pass after pass, it
 // was the critical path of short contexts and of streams past 60 tokens (per
@@ -396,6 +401,7 @@ struct XtLds {
   float xsc[kGQA][32 * NW];     // scores of the pass (base 2)
   float xpw[32 * NW][kGQA];     // softmax numerators, [token][head]
   float2 xred[NW][kGQA][64];    // per-wave value sums
+  float xal[kGQA];              // rescale of the running sums (passes after the first)
 };
 
 template <int NW>
@@ -406,6 +412,7 @@ __device__ __forceinline__ void decode_extras(const SplitParams& p, const int g,
   auto& xsc = L.xsc;
   auto& xpw = L.xpw;
   auto& xred = L.xred;
+  auto& xal = L.xal;
 
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, hh = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -425,8 +432,7 @@ __device__ __forceinline__ void decode_extras(const SplitParams& p, const int g,
   float2 acc[kGQA];
 #pragma unroll
   for (int h = 0; h < kGQA; ++h) acc[h] = make_float2(0.f, 0.f);
-  const int x0 = xi * XT;
-  if (x0 < n_x) {
+  for (int x0 = xi * XT; x0 < n_x; x0 += p.n_xs * XT) {
     const bool mine = col < tw && x0 + tw * w + col < n_x;
     const int xt = min(x0 + tw * w + min(col, tw - 1), n_x - 1);  // clamped: other rows are masked
     int mpos;
@@ -453,7 +459,7 @@ __device__ __forceinline__ void decode_extras(const SplitParams& p, const int g,
       for (int i = 0; i < kGQA; ++i) xsc[i][32 * w + col] = mine ? sacc[i] * sc + madd : -INFINITY;
     }
     __syncthreads();
-    if (w < kGQA) {  // wave w: softmax of head w
+    if (w < kGQA) {  // wave w: online softmax of head w
       float s[XV];
       float mx = -INFINITY;
 #pragma unroll
@@ -461,7 +467,8 @@ __device__ __forceinline__ void decode_extras(const SplitParams& p, const int g,
         s[k] = xsc[w][lane + 64 * k];
         mx = fmaxf(mx, s[k]);
       }
-      m_run = wave64_reduce(mx, OpMax());
+      const float m_old = m_run;
+      m_run = fmaxf(m_old, wave64_reduce(mx, OpMax()));
       float ps = 0.f;
 #pragma unroll
       for (int k = 0; k < XV; ++k) {
@@ -469,9 +476,19 @@ __device__ __forceinline__ void decode_extras(const SplitParams& p, const int g,
         ps += pk;
         xpw[lane + 64 * k][w] = pk;
       }
-      l_run = wave64_reduce(ps, OpAdd());
+      ps = wave64_reduce(ps, OpAdd());
+      const float al = m_run == -INFINITY ? 1.f : fast_exp2(m_old - m_run);
+      l_run = l_run * al + ps;
+      if (lane == 0) xal[w] = al;
     }
     __syncthreads();
+    if (x0 >= p.n_xs * XT) {  // a pass after the workgroup's first
+#pragma unroll
+      for (int h = 0; h < kGQA; ++h) {
+        acc[h].x *= xal[h];
+        acc[h].y *= xal[h];
+      }
+    }
 #pragma unroll
     for (int t = 0; t < 32; ++t) {
       if (t % 4 == 0 && t >= tw) break;
@@ -1630,24 +1647,45 @@ struct RowPlan {
   int n_first, tiles, more, tiles2, more2, two_class, x_at, x_wave;
 };
 
-// Two workgroups per CU in all; the extra tokens take some of them and the
-// compressed tiles the others, as evenly as whole tiles allow.
+// Two workgroups per CU in all (`all` per head); the extra tokens take some of
+// them and the compressed tiles the others, as evenly as whole tiles allow.
+// n_xs is the count whose slower side is the shorter: the tiles of a tile
+// workgroup, or the passes of an extra-token workgroup at kXPassTiles tiles
+// each (one pass a workgroup whatever the tiles are left with: 4 x 2,200 tokens
+// with 1,968 extra 73.4 us, now 22.7; 8 x 1,000 with 668 33.2, now 22.5).  The
+// partial rows per head stay within `all` (twice that where the caller gives
+// the tile splits) or at one more than the tile splits, so a large batch fits
+// the no-allocation scratch with any number of extra tokens.
 inline RowPlan row_plan(const shard_decode_args* a) {
   RowPlan w;
   const int n_tiles = (a->n_comp + kTile - 1) / kTile;
   const int heads = a->n_kv_heads * a->batch, cus = device_cus();
   const int all = (kTG == 1 ? 2 : 1) * cus / heads;
-  auto plan_extras = [&](int x_wave) {
-    const int x_wg = 4 * kTG * x_wave;
-    w.x_wave = x_wave;
-    w.n_xs = (int)((n_extra(a) + x_wg - 1) / x_wg);
-    w.n_t = std::max(1, std::min({a->n_splits > 0 ? a->n_splits : all - w.n_xs, n_tiles, kMaxSplits}));
+  const int room = a->n_splits > 0 ? 2 * all : all;
+  auto ceil_div = [](int x, int y) { return (x + y - 1) / y; };
+  auto tile_splits = [&](int n_xs) {
+    return std::max(1, std::min({a->n_splits > 0 ? a->n_splits : all - n_xs, n_tiles, kMaxSplits}));
   };
-  plan_extras(kXLong);
-  if (n_extra(a) <= kXFew) {
-    const int n_t = w.n_t, per_cu = ((w.n_t + w.n_xs) * heads + cus - 1) / cus;
-    plan_extras(kXShort);
-    if (w.n_t != n_t || ((w.n_t + w.n_xs) * heads + cus - 1) / cus != per_cu) plan_extras(kXLong);
+  auto passes = [&](int x_wave) { return ceil_div((int)n_extra(a), 4 * kTG * x_wave); };
+  const int n_pass = passes(kXLong);
+  w.x_wave = kXLong;
+  w.n_xs = n_pass > 0 ? 1 : 0;
+  int best = 0;
+  for (int n = 1; n <= n_pass && (n == 1 || n + tile_splits(n) <= room); ++n) {
+    const int cost = std::max(ceil_div(n_tiles, tile_splits(n)), kXPassTiles * ceil_div(n_pass, n));
+    if (n == 1 || cost < best) {
+      best = cost;
+      w.n_xs = n;
+    }
+  }
+  w.n_t = tile_splits(w.n_xs);
+  if (n_extra(a) <= kXFew && w.n_xs == n_pass) {
+    const int n_xs = passes(kXShort);
+    if (tile_splits(n_xs) == w.n_t &&
+        ceil_div((w.n_t + n_xs) * heads, cus) == ceil_div((w.n_t + w.n_xs) * heads, cus)) {
+      w.x_wave = kXShort;
+      w.n_xs = n_xs;
+    }
   }
   w.n_splits = w.n_t + w.n_xs;
   w.n_first = w.n_t;
@@ -1945,17 +1983,7 @@ int shard_decode_attn(const shard_decode_args* a, void* workspace, size_t worksp
 int shard_decode_attn_noalloc(const shard_decode_args* a, void* stream) {
   const int st = decode_attn_check(a);
   if (st != SHARD_OK) return st;
-  size_t need = shard_decode_attn_workspace(a);
-  shard_decode_args tok;
-  if (need > SHARD_DECODE_NOALLOC_SCRATCH_BYTES && a->kernel == 0) {
-    // a large batch with many extra tokens: the row-split kernel writes a
-    // partial row per 128 of them and head, the token-tiled one at most about
-    // one per CU and query head of its group
-    tok = *a;
-    tok.kernel = 2;
-    a = &tok;
-    need = shard_decode_attn_workspace(a);
-  }
+  const size_t need = shard_decode_attn_workspace(a);
   if (need > SHARD_DECODE_NOALLOC_SCRATCH_BYTES) {
     char msg[160];
     snprintf(msg, sizeof(msg),

@@ -131,6 +131,25 @@ def test_forced_row_split_beyond_its_extras_runs_token_tiled():
     assert ws(1, 2048 - 67) == ws(2, 2048 - 67)
 
 
+@pytest.mark.parametrize("batch,n_comp,extra", [(1, 8124, 1968), (3, 3000, 1968), (4, 2200, 1968),
+                                                (8, 1000, 1024), (8, 1100, 668), (16, 500, 300),
+                                                (30, 40, 1968), (64, 500, 2048), (200, 30, 2048)])
+def test_row_split_partial_rows_stay_within_the_chip(batch, n_comp, extra):
+    """The row-split kernel's partial rows per head (tile splits and workgroups
+    of extra tokens) fill two workgroups per CU of 256 at most, or are two
+    where that leaves less: the extra tokens take further passes instead of
+    further workgroups, and a large batch keeps within the no-allocation
+    scratch (host-only query)."""
+    from shard_amd import _lib, ops
+    a = _lib.DecodeArgs()
+    a.batch, a.n_q_heads, a.n_kv_heads, a.head_dim, a.rank, a.n_comp = batch, 32, 8, 128, 192, n_comp
+    a.n_sink, a.n_win, a.n_stream, a.kernel = 4, 64, extra - 68, 1
+    need = _lib.load().shard_decode_attn_workspace(ctypes.byref(a))
+    rows, rest = divmod(need, batch * 32 * (128 + 2) * 4)
+    assert rest == 0 and 2 <= rows <= max(2, 512 // (8 * batch))
+    assert need <= ops.DECODE_NOALLOC_SCRATCH_BYTES
+
+
 def test_decode_shapes_and_sizes_on_the_host():
     """Up to 64 query heads per kv head at head_dim 128 (any count: groups of
     4, 3, 2 or 1 per workgroup), and head_dim 64 with an even kv head count

@@ -436,6 +436,37 @@ def test_row_split_extra_workgroups(cuda, B, nkv, n_comp, n_stream, planned):
     assert err <= TOL_ABS and cos >= TOL_COS, (err, cos)
 
 
+@pytest.mark.parametrize("B,nkv,n_comp,n_stream,planned", [
+    (4, 8, 1100, 1200, 1200),   # 10 passes on five workgroups per head
+    (8, 8, 1000, 956, 956),     # 8 on three
+    (16, 8, 500, 232, 232),     # 3 on two, two tile workgroups for 16 tiles
+    (32, 8, 300, 200, 1900),    # one workgroup for all; one for the tiles, ten in turn
+    (32, 8, 60, 0, 1900)])
+def test_row_split_extra_passes(cuda, B, nkv, n_comp, n_stream, planned):
+    """Batches whose extra tokens take several passes per workgroup, down to one
+    tile workgroup per head with many tiles, also where the device counts fewer
+    than planned, against the fp64 oracle."""
+    test_row_split_extra_workgroups(cuda, B, nkv, n_comp, n_stream, planned)
+
+
+def test_row_split_extra_passes_masked(cuda):
+    """Mask rows that hide every token of a workgroup's first pass, of its
+    second, and of both: the passes' online softmax against the fp64 oracle."""
+    B, nkv, n_comp, n_stream = 16, 8, 40, 300
+    gc, inv = random_layer(B=B, nkv=nkv, n_comp=n_comp, n_stream=n_stream, seed=8)
+    q = torch.randn(B, 4 * nkv, 1, 128, generator=torch.Generator().manual_seed(9)).half()
+    total = 4 + n_comp + 64 + n_stream
+    mask = torch.zeros(B, 1, 1, total)
+    low = torch.finfo(torch.float32).min
+    mask[0, ..., :4] = mask[0, ..., 4 + n_comp:n_comp + 128] = low    # the first 128 extra tokens
+    mask[1, ..., n_comp + 128:] = low
+    mask[2, ..., :4] = mask[2, ..., 4 + n_comp:] = low                # all of them
+    want = exact.decode_attention(q.numpy(), gc, nkv, total, inv.numpy(), attn_mask=mask.numpy())
+    got = _run(cuda, gc, inv, q, total, mask=mask.numpy(), nkv=nkv, kernel=1)
+    err, cos = compare(got, want)
+    assert err <= TOL_ABS and cos >= TOL_COS, (err, cos)
+
+
 @pytest.mark.parametrize("rank,nkv,hd", [(160, 8, 128), (320, 8, 128), (512, 4, 128), (320, 8, 64)])
 def test_kv_reconstruct(cuda, rank, nkv, hd):
     """Unfused fp16 reconstruction (_ensure_dequant): V bit-exact, K within fp16
