@@ -66,11 +66,11 @@ constexpr int kTokMaxRank = 256;            // the token-tiled kernel (the row-s
 #define SHARD_SPLIT_PER_XCD 1
 #endif
 constexpr bool kSplitPerXcd = SHARD_SPLIT_PER_XCD;
-// Row-split launches whose (batch row, kv head) groups fill the 8 XCDs evenly
-// put every split of a group on one XCD and run the group's
-// merge workgroups there too, so the merge reads the partial rows that XCD's
-// L2 wrote (8K, batch 1: 13.86 -> 13.51 us).  SHARD_KV_XCD=0 keeps the split
-// order of the other launches.
+// Row-split launches may put every split of a (batch row, kv head) group on one
+// XCD and run the group's merge workgroups there too, so the merge reads the
+// partial rows that XCD's L2 wrote (8K, batch 1: 13.86 -> 13.51 us); every XCD
+// then reads every coefficient row of its batch rows.  kv_xcd_order() holds the
+// line; SHARD_KV_XCD=0 keeps the other launches' split order everywhere.
 #ifndef SHARD_KV_XCD
 #define SHARD_KV_XCD 1
 #endif
@@ -121,9 +121,7 @@ struct SplitParams {
   float* ws_m;
   float* ws_l;
   float* ws_acc;
-  // kv_xcd (launches whose (batch row, kv head) groups fill the 8 XCDs
-  // evenly): every split of a group on one XCD
-  int32_t kv_xcd;
+  int32_t kv_xcd;  // every split of a (batch row, kv head) group on one XCD
 };
 
 // 2^x for the online softmax, where x <= 0 (a difference from the running
@@ -1713,6 +1711,15 @@ inline RowPlan row_plan(const shard_decode_args* a) {
   return w;
 }
 
+// The one-group-per-XCD order, where the groups fill the 8 XCDs evenly.  Time
+// per call against the other order (means over 1 to 20 shapes each): one group
+// per XCD 0.97-0.99; more of them in two classes 0.99 up to 128 groups and 1.035
+// at 256; in one class 1.02-1.03 at 16 to 32 groups, 1.00-1.02 above.
+inline bool kv_xcd_order(const shard_decode_args* a, const RowPlan& w) {
+  const int64_t groups = (int64_t)a->batch * a->n_kv_heads;
+  return SHARD_KV_XCD && groups % 8 == 0 && (groups == 8 || (w.two_class && groups <= 128));
+}
+
 // Token-tiled kernel: the split count and the cost units per split.
 struct TokPlan {
   int n_ct, n_xt, ns, per_u;
@@ -1909,7 +1916,7 @@ static int decode_attn_run(const shard_decode_args* a, void* workspace, hipStrea
   sp.vidx = a->v_idx; sp.vcb = a->v_codebook; sp.vch = a->v_ch;
   sp.mask = a->mask; sp.mask_stride = a->mask_stride; sp.n_sink = a->n_sink;
   sp.ws_m = ws; sp.ws_l = ws + nm; sp.ws_acc = ws + 2 * nm;
-  sp.kv_xcd = SHARD_KV_XCD && (a->batch * a->n_kv_heads) % 8 == 0;
+  sp.kv_xcd = kv_xcd_order(a, pl);
 
   dim3 grid((unsigned)(pl.n_splits * a->n_kv_heads), (unsigned)a->batch);
   switch (a->rank / 16) {
