@@ -39,6 +39,7 @@
 //     of the partial rows, normalized, written as fp16.
 #include <algorithm>
 #include <mutex>
+#include <utility>
 #include <stdio.h>
 
 #include "common.h"
@@ -1558,12 +1559,13 @@ void k_decode_tok(const TokParams p) {
 
 // Which split kernel runs.  The row-split kernel takes query groups of 4 and
 // at most kMaxExtra extra tokens; the token-tiled kernel takes every supported
-// shape.  Automatic choice by the work per CU: the token-tiled kernel has the
-// higher tile throughput but a longer set-up, so it takes over from 9
-// head-tiles per CU (measured on MI355X, row-split vs token-tiled, us per
-// layer-step with append and merge: batch 1 x 8K (7.9 per CU) 17.9 vs 20.1
-// with 268 extra tokens, 20.2 vs 28.4 with 1,968; 1 x 10K (9.9) 19.2 vs 19.2;
-// 1 x 12K 20.8 vs 19.7; 2 x 6K 20.6 vs 19.9; 1 x 16K 22.5 vs 22.2).
+// shape.  Automatic choice: the token-tiled kernel has the higher tile
+// throughput but a longer set-up, so it takes over from 9 head-tiles per CU
+// (measured on MI355X, row-split vs token-tiled, us per layer-step with append
+// and merge: batch 1 x 8K (7.9 per CU) 17.9 vs 20.1 with 268 extra tokens, 20.2
+// vs 28.4 with 1,968; 1 x 10K (9.9) 19.2 vs 19.2; 1 x 12K 20.8 vs 19.7; 2 x 6K
+// 20.6 vs 19.9; 1 x 16K 22.5 vs 22.2), and below that where the row-split plan
+// is the slower one (use_tok).
 constexpr int kTokMinHeadTilesPerCU = 9;
 
 inline int device_cus() {
@@ -1628,21 +1630,11 @@ inline bool split_supported(const shard_decode_args* a) {
          a->rank % 32 == 0 && a->rank <= 192 && n_extra(a) <= kMaxExtra;
 }
 
-// kernel = 1 asks for the row-split kernel; a call it cannot take (query
-// groups other than 4, more than kMaxExtra extra tokens: the reference appends
-// stream tokens without limit, cache.py:156-181) runs on the token-tiled one.
-inline bool use_tok(const shard_decode_args* a) {
-  if (a->kernel == 2) return true;
-  if (a->kernel == 1) return !split_supported(a);
-  if (!split_supported(a)) return true;
-  const int64_t tiles = (int64_t)((a->n_comp + kTile - 1) / kTile) * a->n_kv_heads * a->batch;
-  return tiles >= (int64_t)kTokMinHeadTilesPerCU * device_cus();
-}
-
 // Row-split kernel: the workgroups of a (batch row, kv head).
 struct RowPlan {
   int n_t, n_xs, n_splits;  // tile splits, extra-token splits, both
   int n_first, tiles, more, tiles2, more2, two_class, x_at, x_wave;
+  int cost, cost_empty;  // in tiles; cost_empty: with no stream rows yet
 };
 
 // Two workgroups per CU in all (`all` per head); the extra tokens take some of
@@ -1650,7 +1642,7 @@ struct RowPlan {
 // n_xs is the count whose slower side is the shorter: the tiles of a tile
 // workgroup, or the passes of an extra-token workgroup at kXPassTiles tiles
 // each (one pass a workgroup whatever the tiles are left with: 4 x 2,200 tokens
-// with 1,968 extra 73.4 us, now 22.7; 8 x 1,000 with 668 33.2, now 22.5).  The
+// with 1,968 extra 73.4 us, now 21.5; 8 x 1,000 with 668 33.2, now 22.2).  The
 // partial rows per head stay within `all` (twice that where the caller gives
 // the tile splits) or at one more than the tile splits, so a large batch fits
 // the no-allocation scratch with any number of extra tokens.
@@ -1668,9 +1660,10 @@ inline RowPlan row_plan(const shard_decode_args* a) {
   const int n_pass = passes(kXLong);
   w.x_wave = kXLong;
   w.n_xs = n_pass > 0 ? 1 : 0;
-  int best = 0;
+  std::pair<int, int> best;  // the slower side, then both
   for (int n = 1; n <= n_pass && (n == 1 || n + tile_splits(n) <= room); ++n) {
-    const int cost = std::max(ceil_div(n_tiles, tile_splits(n)), kXPassTiles * ceil_div(n_pass, n));
+    const int t = ceil_div(n_tiles, tile_splits(n)), x = kXPassTiles * ceil_div(n_pass, n);
+    const std::pair<int, int> cost(std::max(t, x), t + x);
     if (n == 1 || cost < best) {
       best = cost;
       w.n_xs = n;
@@ -1708,6 +1701,12 @@ inline RowPlan row_plan(const shard_decode_args* a) {
       w.x_at = w.n_t;  // the last workgroups of the second class
     }
   }
+  // the fullest tile workgroup (two classes finish together) and the passes
+  const int fixed = ceil_div((int)(n_extra(a) - a->n_stream), 4 * kTG * kXLong);
+  const int t_cost = w.two_class ? (n_tiles + w.n_t / 2) / w.n_t : ceil_div(n_tiles, w.n_t);
+  const int x_wgs = std::max(w.n_xs, 1);
+  w.cost = std::max(t_cost, kXPassTiles * ceil_div(passes(w.x_wave), x_wgs));
+  w.cost_empty = std::max(t_cost, kXPassTiles * ceil_div(fixed, x_wgs));
   return w;
 }
 
@@ -1742,6 +1741,40 @@ inline TokPlan tok_plan(const shard_decode_args* a) {
   w.per_u = (int)std::max<int64_t>(per, 1);
   w.ns = (int)((U + w.per_u - 1) / w.per_u);
   return w;
+}
+
+// kernel = 1 asks for the row-split kernel; a call it cannot take (query
+// groups other than 4, more than kMaxExtra extra tokens: the reference appends
+// stream tokens without limit, cache.py:156-181) runs on the token-tiled one.
+// Below kTokMinHeadTilesPerCU both plans' costs decide, fitted to 210 shapes
+// (batch 1 to 48, 1 to 8 kv heads, 69 to 2,040 extra tokens, every layer cold):
+// row-split minus token-tiled in us = 0.86 x the row plan's cost - 0.28 x the
+// extra tiles of the token-tiled plan's fullest split - 2.2 x its rounds of
+// workgroups after the first - 3.1.  The choice is within 3 % of the faster
+// kernel at 203 of them; a cut at 256 extra tokens at 108.  Row-split against
+// token-tiled, us: 4 x 2,200 tokens with 1,968 extra 21.8 and 28.1, with 78 14.9 and 14.6;
+// 8 x 1,000 with 1,024 23.2 and 31.3; 16 x 500 with 300 21.6 and 19.5;
+// 32 x 250 with 78 23.9 and 19.1.  A merge of more than 128 partial rows is slow
+// (one kv head, 39,712 tokens: 46.9 and 28.3).
+// A stream that the device counts may hold anything from none of its n_stream
+// rows to all: the cost at both ends counts, the tiles then for more, since the
+// workgroups planned for the extra tokens stand idle at first (planned for
+// 1,968, 68 there: 4 x 2,200 21.3 and 14.2, 1 x 8,124 13.9 and 13.5).
+inline bool use_tok(const shard_decode_args* a) {
+  if (a->kernel == 2) return true;
+  if (a->kernel == 1) return !split_supported(a);
+  if (!split_supported(a)) return true;
+  const int64_t tiles = (int64_t)((a->n_comp + kTile - 1) / kTile) * a->n_kv_heads * a->batch;
+  if (tiles >= (int64_t)kTokMinHeadTilesPerCU * device_cus()) return true;
+  const RowPlan row = row_plan(a);
+  if (row.n_splits > 128) return true;
+  const TokPlan tok = tok_plan(a);
+  const int64_t wgs = (int64_t)tok.ns * a->n_kv_heads * a->batch;  // 4 query heads per kv head
+  const int64_t later = (wgs - 1) / device_cus();                  // rounds after the first
+  const int64_t tok_x = std::min(tok.n_xt, tok.per_u);
+  if (a->n_stream_dev && n_extra(a) > kXFew)
+    return 3 * row.cost + 5 * row.cost_empty > 26 + tok_x + 16 * later;
+  return 3 * row.cost > 10 + tok_x + 8 * later;
 }
 
 template <int KS>

@@ -150,6 +150,32 @@ def test_row_split_partial_rows_stay_within_the_chip(batch, n_comp, extra):
     assert need <= ops.DECODE_NOALLOC_SCRATCH_BYTES
 
 
+@pytest.mark.parametrize("batch,n_kv,n_comp,extra,want,want_counted", [
+    (1, 8, 1980, 132, 1, 1), (1, 8, 2000, 1968, 1, 1), (1, 8, 8124, 268, 1, 1),
+    (1, 8, 12000, 78, 2, 2), (2, 8, 4400, 1968, 1, 1), (4, 8, 2200, 1968, 1, 2),
+    (8, 8, 1000, 1024, 1, 2), (16, 8, 500, 300, 2, 2), (32, 8, 250, 78, 2, 2),
+    (30, 8, 40, 1968, 2, 2), (1, 1, 39712, 1304, 2, 2)])
+def test_automatic_kernel_choice_by_both_plans(batch, n_kv, n_comp, extra, want, want_counted):
+    """The kernel an automatic call is planned on: the row-split one unless its
+    extra tokens or a large batch leave the tiles too few workgroups, with the
+    stream's rows known to the host, then counted by the device (planned, but
+    perhaps not there yet).  Host-only queries."""
+    from shard_amd import _lib
+    lib = _lib.load()
+
+    def ws(kernel, counted):
+        a = _lib.DecodeArgs()
+        a.batch, a.n_q_heads, a.n_kv_heads, a.head_dim = batch, 4 * n_kv, n_kv, 128
+        a.rank, a.n_comp = 192, n_comp
+        a.n_sink, a.n_win, a.n_stream, a.kernel = 4, 64, extra - 68, kernel
+        a.n_stream_dev = 16 if counted else None
+        return lib.shard_decode_attn_workspace(ctypes.byref(a))
+
+    for counted, k in ((False, want), (True, want_counted)):
+        assert ws(1, counted) != ws(2, counted)
+        assert ws(0, counted) == ws(k, counted), counted
+
+
 def test_decode_shapes_and_sizes_on_the_host():
     """Up to 64 query heads per kv head at head_dim 128 (any count: groups of
     4, 3, 2 or 1 per workgroup), and head_dim 64 with an even kv head count

@@ -449,6 +449,20 @@ def test_row_split_extra_passes(cuda, B, nkv, n_comp, n_stream, planned):
     test_row_split_extra_workgroups(cuda, B, nkv, n_comp, n_stream, planned)
 
 
+@pytest.mark.parametrize("B,nkv,n_comp,n_stream", [
+    (4, 8, 1100, 1200), (8, 8, 1000, 600), (3, 8, 1600, 1900), (16, 8, 500, 232), (32, 8, 250, 10)])
+def test_automatic_choice_with_many_extra_tokens(cuda, B, nkv, n_comp, n_stream):
+    """The automatic choice (row-split for the first three, token-tiled for the
+    others) on batches whose extra tokens compete with the tiles for
+    workgroups, against the fp64 oracle."""
+    gc, inv = random_layer(B=B, nkv=nkv, n_comp=n_comp, n_stream=n_stream, seed=n_comp + B)
+    q = torch.randn(B, 4 * nkv, 1, 128, generator=torch.Generator().manual_seed(6)).half()
+    pos_q = 4 + n_comp + 64 + n_stream
+    want = exact.decode_attention(q.numpy(), gc, nkv, pos_q, inv.numpy())
+    err, cos = compare(_run(cuda, gc, inv, q, pos_q, nkv=nkv), want)
+    assert err <= TOL_ABS and cos >= TOL_COS, (err, cos)
+
+
 def test_row_split_extra_passes_masked(cuda):
     """Mask rows that hide every token of a workgroup's first pass, of its
     second, and of both: the passes' online softmax against the fp64 oracle."""
