@@ -625,10 +625,14 @@ class _EigJob:
     for orthogonality and residual.  A layer that misses the bounds (clustered
     or zero eigenvalues, a non-finite covariance), is larger than the kernel
     takes or is asked for more pairs than it has (it gives them all) goes to
-    the host's float64 eigh, errors included."""
+    the host's float64 eigh, errors included; on_gpu says after result() which
+    one it was.  Both read the lower triangle: a GEMM's two triangles may
+    differ in their last bits (split sums: 1e-6 of the largest entry at p = 512
+    from 32,768 rows on)."""
 
     def __init__(self, cov: torch.Tensor, rank: int):
         self.cov, self.rank = cov.detach(), rank
+        self.on_gpu = False
         self.future = None
         p = cov.shape[0]
         if not cov.is_cuda or not 2 <= p <= ops.EIGH_MAX or not 1 <= rank <= p:
@@ -642,7 +646,8 @@ class _EigJob:
     @torch.no_grad()
     def _solve(self):
         with torch.cuda.device(self.cov.device), torch.cuda.stream(self.side):
-            cov = self.cov.double()
+            low = self.cov.double().tril()
+            cov = low + low.tril(-1).t()
             evals, evecs = ops.eigh_top(cov, self.rank)
             gram = evecs @ evecs.t().contiguous()
             gram.diagonal().sub_(1.0)
@@ -659,6 +664,7 @@ class _EigJob:
             stat.record_stream(self.main)
             host_stat = stat.cpu()
             if host_stat[0] <= _EIG_ORTH and host_stat[1] <= _EIG_RESID:  # False for NaN
+                self.on_gpu = True
                 return evecs.float().t(), host_stat[2:].clamp(min=0.0).float()
         basis, eig = _eigh_top(self.cov.double().cpu(), self.rank)
         return basis.to(self.cov.device), eig
@@ -727,6 +733,8 @@ def compress_layer(cache: Cache, k_full: torch.Tensor, v_full: torch.Tensor, li:
     del x
     if eig_job is not None:
         basis, eig = eig_job.result()
+        if not eig_job.on_gpu:  # counted: such a layer takes the host's eigensolver
+            cache._pca_host_solves = getattr(cache, "_pca_host_solves", 0) + 1
     budget = max(64, int(p_dim * 16 / cache._k_target_cr))
     alloc = host.dp_bit_allocation(eig, budget)
     keep = sum(1 for b in alloc if b > 0)

@@ -171,12 +171,12 @@ def _centred_rows(k, inv, sink=4, win=64):
 
 def test_production_pca_basis_matches_exact_svd(cuda):
     """The basis Cache.compress takes without a supplied one (fp32 covariance
-    of the fp32 centred rows on the GPU, float64 eigh on the host) against the
+    of the fp32 centred rows and float64 eigensolver, both on the GPU) against the
     float64 SVD of the same rows on the CPU (the quantities svd_lowrank
     approximates, cache.py:376-378): principal angles of the top-keep subspace,
     the variances S^2 / n, and the same dp_bit_allocation."""
     from shard_amd import bench_data, host, ops
-    from shard_amd.cache import _covariance, pca_basis_cov, _undo_rope_mean
+    from shard_amd.cache import _EigJob, _covariance, _undo_rope_mean
     k, _ = bench_data.make_kv(2048)
     inv = bench_data.inv_freq()
     x = _centred_rows(k, inv).double()
@@ -186,7 +186,9 @@ def test_production_pca_basis_matches_exact_svd(cuda):
     kd = k.to(cuda)
     mean = _undo_rope_mean(kd, 4, 2048 - 64, inv)
     centered = ops.k_prepare(kd, 4, 2048 - 68, inv.to(cuda), mean, out_dtype=torch.float32)
-    basis, ev = pca_basis_cov(_covariance(centered), 192)
+    job = _EigJob(_covariance(centered), 192)
+    basis, ev = job.result()
+    assert job.on_gpu
     basis, ev = basis.cpu().double(), ev.cpu().double()
     rel = float(((ev - ev_want).abs() / ev_want).max())
     budget = max(64, int(1024 * 16 / 20.0))
@@ -348,6 +350,38 @@ def test_eig_job_hands_clusters_and_bad_input_to_the_host(cuda):
         want, eig_want = _eigh_top(c.double(), 20)
         assert torch.equal(basis.cpu().nan_to_num(7.0), want.nan_to_num(7.0))
         assert torch.equal(eig.cpu().nan_to_num(7.0), eig_want.nan_to_num(7.0))
+
+
+def _spectrum_cov(p, spectrum, seed=0):
+    """A symmetric float64 (p, p) matrix with the given eigenvalues."""
+    q, _ = torch.linalg.qr(torch.randn(p, p, generator=torch.Generator().manual_seed(seed),
+                                       dtype=torch.float64))
+    c = (q * spectrum) @ q.T
+    return (c + c.T) / 2
+
+
+def test_eig_job_reads_one_triangle(cuda, monkeypatch):
+    """A covariance whose triangles differ in their last fp32 bits (a GEMM that
+    groups their sums differently) is solved on the GPU, from its lower
+    triangle as the host's eigh: the same basis up to the vectors' signs."""
+    from shard_amd import cache
+    p = 512
+    c = _spectrum_cov(p, torch.exp(-torch.arange(p, dtype=torch.float64) / 100)).float()
+    noise = torch.randn(p, p, generator=torch.Generator().manual_seed(1)).triu(1)
+    c += 1e-6 * noise
+    want, eig_want = cache._eigh_top(c.double(), 64)
+
+    def no_host(*_):
+        raise AssertionError("the host's eigensolver was called")
+    monkeypatch.setattr(cache, "_eigh_top", no_host)
+    job = cache._EigJob(c.to(cuda), 64)
+    basis, eig = job.result()
+    assert job.on_gpu
+    basis = basis.cpu()
+    sign = (basis.double() * want.double()).sum(0).sign().float()
+    # float64 vectors 1e-13 apart, rounded to fp32
+    assert float((basis * sign - want).abs().max()) <= 2.0 ** -24
+    assert float((eig.cpu() - eig_want).abs().max()) <= 2.0 ** -23
 
 
 def test_pca_basis_cov_of_fewer_columns_than_asked(cuda):
