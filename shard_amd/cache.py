@@ -611,6 +611,20 @@ def _host_worker():
     return _host_pool
 
 
+# The eigensolver's stream on each device, one for the process: the one worker
+# above takes the jobs in turn anyway, and the allocator keeps a stream's freed
+# blocks (170 MiB of float64 matrices and BLAS workspace at p = 1024) for that
+# stream alone.
+_side_streams = {}
+
+
+def _side_stream(device):
+    stream = _side_streams.get(device)
+    if stream is None:
+        stream = _side_streams.setdefault(device, torch.cuda.Stream(device))
+    return stream
+
+
 # Bounds an eigensolve on the GPU has to meet (float64 sums of the float32
 # basis it gives are not affected below them): orthogonality of the vectors,
 # residual relative to the largest eigenvalue.
@@ -638,7 +652,7 @@ class _EigJob:
         if not cov.is_cuda or not 2 <= p <= ops.EIGH_MAX or not 1 <= rank <= p:
             return
         self.main = torch.cuda.current_stream(cov.device)
-        self.side = torch.cuda.Stream(cov.device)
+        self.side = _side_stream(cov.device)
         self.side.wait_stream(self.main)
         self.cov.record_stream(self.side)
         self.future = _host_worker().submit(self._solve)

@@ -384,6 +384,21 @@ def test_eig_job_reads_one_triangle(cuda, monkeypatch):
     assert float((eig.cpu() - eig_want).abs().max()) <= 2.0 ** -23
 
 
+def test_eig_jobs_share_their_memory(cuda):
+    """The layers of a model are solved one after another in the same device
+    memory: after the first two jobs, further ones reserve none."""
+    from shard_amd.cache import _EigJob
+    c = torch.diag(torch.linspace(2, 1, 1024)).to(cuda)
+    for _ in range(2):
+        _EigJob(c, 192).result()
+    torch.cuda.synchronize()
+    held = torch.cuda.memory_reserved()
+    for _ in range(8):
+        _EigJob(c, 192).result()
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_reserved() <= held
+
+
 def test_pca_basis_cov_of_fewer_columns_than_asked(cuda):
     """More eigenpairs than the covariance has gives them all, on either device."""
     from shard_amd.cache import pca_basis_cov
