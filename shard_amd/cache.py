@@ -23,6 +23,7 @@ import torch
 from transformers.cache_utils import Cache as HFCache, CacheLayerMixin
 
 from . import host, ops
+from ._lib import ShardHipUnavailable
 
 
 def _nb(t):
@@ -602,8 +603,8 @@ _host_pool = None
 
 
 def _host_worker():
-    """One background thread for host work beside the caller's (the launches of
-    the PCA eigendecomposition, while the V codec's are issued)."""
+    """One background thread for host work beside the caller's (the PCA
+    eigendecomposition, while the V codec's kernels are issued and run)."""
     global _host_pool
     if _host_pool is None:
         import concurrent.futures
@@ -632,56 +633,68 @@ _EIG_ORTH, _EIG_RESID = 1e-8, 1e-10
 
 
 class _EigJob:
-    """The top-`rank` eigenpairs of a (p, p) covariance, solved on a side
-    stream while the caller's stream goes on: shard_eigh_top in float64 (6.6 ms
-    at p = 1024, most of it the 1,023 launches of the tridiagonalization, which
-    a background thread issues; LAPACK on the host took 50 to 200 ms), checked
-    for orthogonality and residual.  A layer that misses the bounds (clustered
-    or zero eigenvalues, a non-finite covariance), is larger than the kernel
-    takes or is asked for more pairs than it has (it gives them all) goes to
-    the host's float64 eigh, errors included; on_gpu says after result() which
-    one it was.  Both read the lower triangle: a GEMM's two triangles may
-    differ in their last bits (split sums: 1e-6 of the largest entry at p = 512
-    from 32,768 rows on)."""
+    """The top-`rank` eigenpairs of a (p, p) covariance, solved beside the
+    caller: shard_eigh_top in float64 on a side stream (6.6 ms at p = 1024, most
+    of it the 1,023 launches of the tridiagonalization, which the background
+    thread issues; LAPACK on the host took 50 to 200 ms), checked for
+    orthogonality and residual.  A layer that misses the bounds (clustered or
+    zero eigenvalues, a non-finite covariance) or whose solve fails (out of
+    device memory), that is larger than the kernel takes or is asked for more
+    pairs than it has (it gives them all) goes to the host's float64 eigh on the same
+    thread, errors included; on_gpu says after result() which one it was, error
+    holds a failed solve's exception.  Both read the lower triangle: a GEMM's
+    two triangles may differ in their last bits (split sums: 1e-6 of the largest
+    entry at p = 512 from 32,768 rows on)."""
 
     def __init__(self, cov: torch.Tensor, rank: int):
         self.cov, self.rank = cov.detach(), rank
-        self.on_gpu = False
-        self.future = None
-        p = cov.shape[0]
-        if not cov.is_cuda or not 2 <= p <= ops.EIGH_MAX or not 1 <= rank <= p:
-            return
-        self.main = torch.cuda.current_stream(cov.device)
-        self.side = _side_stream(cov.device)
-        self.side.wait_stream(self.main)
-        self.cov.record_stream(self.side)
+        self.on_gpu, self.error = False, None
+        if cov.is_cuda:
+            self.side = _side_stream(cov.device)
+            self.side.wait_stream(torch.cuda.current_stream(cov.device))
+            self.cov.record_stream(self.side)
         self.future = _host_worker().submit(self._solve)
 
     @torch.no_grad()
     def _solve(self):
+        """(basis, eigenvalues on the host) on the worker, which waits for the
+        side stream where the caller does not."""
+        if not self.cov.is_cuda:
+            return _eigh_top(self.cov.double(), self.rank)
         with torch.cuda.device(self.cov.device), torch.cuda.stream(self.side):
-            low = self.cov.double().tril()
-            cov = low + low.tril(-1).t()
-            evals, evecs = ops.eigh_top(cov, self.rank)
-            gram = evecs @ evecs.t().contiguous()
-            gram.diagonal().sub_(1.0)
-            vt = evecs.t().contiguous()
-            resid = (cov @ vt - vt * evals).abs().max() / evals[0].abs()
-            return evecs, torch.cat([torch.stack([gram.abs().max(), resid]), evals])
+            if 2 <= self.cov.shape[0] <= ops.EIGH_MAX and 1 <= self.rank <= self.cov.shape[0]:
+                try:
+                    found = self._solve_gpu()
+                except ShardHipUnavailable:
+                    raise
+                except RuntimeError as exc:  # without the frames, which hold device tensors
+                    self.error, found = exc.with_traceback(None), None
+                if found is not None:
+                    self.on_gpu = True
+                    return found
+            return _eigh_top(self.cov.cpu().double(), self.rank)
+
+    def _solve_gpu(self):
+        low = self.cov.double().tril()
+        cov = low + low.tril(-1).t()
+        evals, evecs = ops.eigh_top(cov, self.rank)
+        gram = evecs @ evecs.t().contiguous()
+        gram.diagonal().sub_(1.0)
+        vt = evecs.t().contiguous()
+        resid = (cov @ vt - vt * evals).abs().max() / evals[0].abs()
+        stat = torch.cat([torch.stack([gram.abs().max(), resid]), evals]).cpu()
+        if not (stat[0] <= _EIG_ORTH and stat[1] <= _EIG_RESID):  # True for NaN
+            return None
+        return evecs, stat[2:].clamp(min=0.0).float()
 
     def result(self):
-        """(basis (p, rank) fp32 on the device, eigenvalues (rank) fp32)."""
-        if self.future is not None:
-            evecs, stat = self.future.result()
-            self.main.wait_stream(self.side)
-            evecs.record_stream(self.main)
-            stat.record_stream(self.main)
-            host_stat = stat.cpu()
-            if host_stat[0] <= _EIG_ORTH and host_stat[1] <= _EIG_RESID:  # False for NaN
-                self.on_gpu = True
-                return evecs.float().t(), host_stat[2:].clamp(min=0.0).float()
-        basis, eig = _eigh_top(self.cov.double().cpu(), self.rank)
-        return basis.to(self.cov.device), eig
+        """(basis (p, rank) fp32 on the covariance's device, eigenvalues (rank)
+        fp32 on the host)."""
+        found, eig = self.future.result()
+        if self.on_gpu:  # (rank, p) float64 of the side stream, which is through
+            found.record_stream(torch.cuda.current_stream(found.device))
+            return found.float().t(), eig
+        return found.to(self.cov.device), eig
 
 
 def pca_basis_cov(cov: torch.Tensor, rank: int):

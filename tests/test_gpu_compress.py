@@ -384,6 +384,33 @@ def test_eig_job_reads_one_triangle(cuda, monkeypatch):
     assert float((eig.cpu() - eig_want).abs().max()) <= 2.0 ** -23
 
 
+def test_eig_job_falls_back_beside_the_caller(cuda, monkeypatch):
+    """The host's solve of a layer that the GPU's misses, cannot take or fails
+    on runs on the background thread, and a failed GPU solve is no error."""
+    import threading
+    from shard_amd import cache
+    seen = []
+    host = cache._eigh_top
+
+    def recording(*args):
+        seen.append(threading.current_thread().name)
+        return host(*args)
+    monkeypatch.setattr(cache, "_eigh_top", recording)
+    for c in (torch.eye(96), torch.diag(torch.arange(1.0, 1031.0))):
+        cache._EigJob(c.to(cuda), 20).result()
+    assert len(seen) == 2 and all(n.startswith("shard-host") for n in seen)
+
+    def no_memory(*_):
+        raise torch.OutOfMemoryError("no memory")
+    monkeypatch.setattr(cache.ops, "eigh_top", no_memory)
+    c = _spectrum_cov(64, torch.arange(64.0, 0.0, -1.0, dtype=torch.float64)).float()
+    job = cache._EigJob(c.to(cuda), 20)
+    basis, eig = job.result()
+    want, eig_want = host(c.double(), 20)
+    assert not job.on_gpu and isinstance(job.error, torch.OutOfMemoryError)
+    assert torch.equal(basis.cpu(), want) and torch.equal(eig, eig_want)
+
+
 def test_eig_jobs_share_their_memory(cuda):
     """The layers of a model are solved one after another in the same device
     memory: after the first two jobs, further ones reserve none."""
