@@ -626,10 +626,17 @@ def _side_stream(device):
     return stream
 
 
-# Bounds an eigensolve on the GPU has to meet (float64 sums of the float32
-# basis it gives are not affected below them): orthogonality of the vectors,
-# residual relative to the largest eigenvalue.
-_EIG_ORTH, _EIG_RESID = 1e-8, 1e-10
+# Bounds an eigensolve on the GPU has to meet: orthogonality of the vectors,
+# residual relative to the largest eigenvalue.  Two vectors a relative gap g
+# apart may be turned into each other by up to residual / g: measured residuals
+# are 2e-16 to 7e-16 (flat, exponential, power-law and nearly equal spectra,
+# orders 64 to 1,024), LAPACK's on the same matrices 2e-16 to 1.4e-15, so the
+# bound grants no more than ten times a library's own.  The orthogonality is
+# 1e-14 to 4e-12 on covariances and 3e-10 at gaps near 1e-8; past that the
+# vectors of close eigenvalues collapse (0.01 and more).  The bound lies at
+# the fp32 rounding of the basis (2^-25 of elements of about 1 / sqrt(p): 1e-9
+# in an inner product of order 1,024).
+_EIG_ORTH, _EIG_RESID = 1e-9, 1e-14
 
 
 class _EigJob:

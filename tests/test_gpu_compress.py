@@ -411,6 +411,32 @@ def test_eig_job_falls_back_beside_the_caller(cuda, monkeypatch):
     assert torch.equal(basis.cpu(), want) and torch.equal(eig, eig_want)
 
 
+def test_eig_job_refuses_turned_vectors(cuda, monkeypatch):
+    """Two vectors of eigenvalues 1e-6 apart turned into each other by 1e-5 are
+    orthogonal with a residual of 1e-11: not what a float64 eigensolver gives,
+    so the host solves."""
+    from shard_amd import cache
+    p = 96
+    spectrum = torch.cat([torch.tensor([1.0, 1.0 - 1e-6], dtype=torch.float64),
+                          torch.linspace(0.5, 0.1, p - 2, dtype=torch.float64)])
+    # float32 entries, as a covariance's: the eigenvalues move by 1e-8
+    c = _spectrum_cov(p, spectrum).float().to(cuda)
+    solve = cache.ops.eigh_top
+
+    def turned(a, top):
+        w, v = solve(a, top)
+        v[0], v[1] = v[0] + 1e-5 * v[1], v[1] - 1e-5 * v[0]
+        return w, v
+    job = cache._EigJob(c, 20)
+    job.result()
+    assert job.on_gpu
+    monkeypatch.setattr(cache.ops, "eigh_top", turned)
+    job = cache._EigJob(c, 20)
+    basis, _ = job.result()
+    assert not job.on_gpu
+    assert torch.equal(basis.cpu(), cache._eigh_top(c.cpu().double(), 20)[0])
+
+
 def test_eig_jobs_share_their_memory(cuda):
     """The layers of a model are solved one after another in the same device
     memory: after the first two jobs, further ones reserve none."""
