@@ -876,10 +876,31 @@ def test_pca_project_rope_few_rows(cuda, B, G, T, n, start, n_comp):
     got = ops.pca_project_rope(k, start, n_comp, ph, ops.rope_basis(bt), bias)
     a = ops.k_prepare(k, start, n_comp, inv, torch.zeros(G * 128, device=cuda))
     want = a.double() @ bt.double().t().contiguous() - bias.double()
-    # fp32 sums of G * 128 products: about sqrt(k) ulps of their magnitude
-    tol = 1e-6 * (G * 128) ** 0.5 * float((a.double().abs() @ bt.double().abs().t().contiguous()).max())
+    # fp32 sums of exact fp16 products, 16 a step (G * 8 steps and the tree inside
+    # one), then the bias: half an ulp of the products' magnitude for each
+    mag = a.double().abs() @ bt.double().abs().t().contiguous() + bias.double().abs()
     assert got.shape == (B * n_comp, n)
-    assert float((got.double() - want).abs().max()) <= tol
+    assert float(((got.double() - want).abs() / mag).max()) <= (G * 8 + 6) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n", [32, 192, 256])
+def test_pca_project_rope_same_bits_at_any_row_count(cuda, n):
+    """A token's projection has the same bits whichever kernel its batch's row
+    count selects (blocks of C, 32, 64 and 128 rows per workgroup): the int4
+    codes of a prompt do not depend on its neighbours in the batch."""
+    from shard_amd import bench_data, ops
+    g = torch.Generator().manual_seed(n)
+    G, T, start, n_comp = 8, 310, 4, 300
+    k = torch.randn(1, G, T, 128, generator=g).half().to(cuda)
+    basis = ops.rope_basis((torch.randn(n, G * 128, generator=g) / 32).half().to(cuda))
+    bias = torch.randn(n, generator=g).to(cuda)
+    ph = ops.rope_phases(start, n_comp, bench_data.inv_freq().to(cuda))
+    # 300, 4,500 and 12,000 rows (at most 256 tiles of 32 or 64), 18,000 (more)
+    got = [ops.pca_project_rope(k.expand(B, -1, -1, -1).contiguous(), start, n_comp, ph, basis, bias)
+           for B in (1, 15, 40, 60)]
+    for B, c in zip((1, 15, 40, 60), got):
+        for b in (0, B - 1):
+            assert torch.equal(c[b * n_comp:(b + 1) * n_comp], got[3][:n_comp]), (B, b)
 
 
 @pytest.mark.parametrize("n", [1, 63, 256, 100003])
