@@ -1642,7 +1642,7 @@ struct RowPlan {
 // n_xs is the count whose slower side is the shorter: the tiles of a tile
 // workgroup, or the passes of an extra-token workgroup at kXPassTiles tiles
 // each (one pass a workgroup whatever the tiles are left with: 4 x 2,200 tokens
-// with 1,968 extra 73.4 us, now 21.5; 8 x 1,000 with 668 33.2, now 22.2).  The
+// with 1,968 extra 73.4 us, now 20.4; 8 x 1,000 with 668 33.2, now 20.7).  The
 // partial rows per head stay within `all` (twice that where the caller gives
 // the tile splits) or at one more than the tile splits, so a large batch fits
 // the no-allocation scratch with any number of extra tokens.
@@ -1688,17 +1688,24 @@ inline RowPlan row_plan(const shard_decode_args* a) {
   // the class split assumes 256 CUs (two classes of 256 workgroups)
   if (kTG == 1 && kSplitBias && device_cus() == 256 &&
       (int64_t)w.n_splits * a->n_kv_heads * a->batch == 512 && w.n_splits % 2 == 0 &&
-      32 % a->n_kv_heads == 0 && n_tiles >= 2 * w.n_splits && rest > 0) {
-    const int ta = (97 * half + 64 * n_tiles) / (100 * half);  // round(0.47 + 0.64 n_tiles / half)
-    const int left = n_tiles - half * ta;
-    if (ta >= 1 && left >= rest) {
+      32 % a->n_kv_heads == 0 && n_tiles >= 2 * w.n_splits && rest >= 0) {
+    // The second class holds `rest` tile workgroups beside the extra tokens'.
+    // One with tb = (ta - 0.47) / 0.64 - ta tiles ends with a first-class one
+    // of ta, so ta = (n_tiles + 0.73 rest) / (half + 0.56 rest), rounded.  As
+    // if the second class were all tiles, it left a few workgroups there too
+    // many: 16 x 280 tokens with 78 extra 15.4 us, now 14.2; 32 x 100 with 78
+    // 19.1, now 16.6; 8 x 1,100 with 668 24.6, now 21.0.
+    w.two_class = 1;
+    w.x_at = w.n_t;  // the last workgroups of the second class
+    if (rest > 0) {
+      const int num = 100 * n_tiles + 73 * rest, den = 100 * half + 56 * rest;
+      const int ta = std::max(1, std::min((2 * num + den) / (2 * den), (n_tiles - rest) / half));
+      const int left = n_tiles - half * ta;  // >= rest
       w.n_first = half;
       w.tiles = ta;
       w.more = 0;
       w.tiles2 = left / rest;
       w.more2 = left % rest;
-      w.two_class = 1;
-      w.x_at = w.n_t;  // the last workgroups of the second class
     }
   }
   // the fullest tile workgroup (two classes finish together) and the passes
@@ -1750,11 +1757,10 @@ inline TokPlan tok_plan(const shard_decode_args* a) {
 // (batch 1 to 48, 1 to 8 kv heads, 69 to 2,040 extra tokens, every layer cold):
 // row-split minus token-tiled in us = 0.86 x the row plan's cost - 0.28 x the
 // extra tiles of the token-tiled plan's fullest split - 2.2 x its rounds of
-// workgroups after the first - 3.1.  The choice is within 3 % of the faster
-// kernel at 203 of them; a cut at 256 extra tokens at 108.  Row-split against
-// token-tiled, us: 4 x 2,200 tokens with 1,968 extra 21.8 and 28.1, with 78 14.9 and 14.6;
-// 8 x 1,000 with 1,024 23.2 and 31.3; 16 x 500 with 300 21.6 and 19.5;
-// 32 x 250 with 78 23.9 and 19.1.  A merge of more than 128 partial rows is slow
+// workgroups after the first - 3.1.  At 157 other shapes the choice is 0.3 %
+// from the faster kernel on average, more than 3 % at 8.  Row-split against
+// token-tiled, us: 4 x 2,200 tokens with 1,968 extra 20.2 and 28.4, with 78 14.9
+// and 14.8; 8 x 1,000 with 1,024 22.0 and 31.6; 32 x 250 with 78 20.5 and 19.6.  A merge of more than 128 partial rows is slow
 // (one kv head, 39,712 tokens: 46.9 and 28.3).
 // A stream that the device counts may hold anything from none of its n_stream
 // rows to all: the cost at both ends counts, the tiles then for more, since the
