@@ -481,7 +481,7 @@ int shard_kv_rebuild(const shard_decode_args* args, uint16_t* k_out,
  * 1024, which is overwritten: the PCA basis of a layer's key covariance
  * (svd_lowrank of cache.py:376-378, exactly and deterministically).
  * Householder tridiagonalization, Sturm multisection, twisted factorizations.
- * Vectors of nearly equal eigenvalues (closer than about 1e-6 of the largest)
+ * Vectors of nearly equal eigenvalues (closer than about 1e-7 of the largest)
  * are not reorthogonalized, and non-finite input gives non-finite output:
  * check V V^T and the residual before use. */
 size_t shard_eigh_top_workspace(int32_t n);

@@ -1760,12 +1760,13 @@ inline TokPlan tok_plan(const shard_decode_args* a) {
 // workgroups after the first - 3.1.  At 157 other shapes the choice is 0.3 %
 // from the faster kernel on average, more than 3 % at 8.  Row-split against
 // token-tiled, us: 4 x 2,200 tokens with 1,968 extra 20.2 and 28.4, with 78 14.9
-// and 14.8; 8 x 1,000 with 1,024 22.0 and 31.6; 32 x 250 with 78 20.5 and 19.6.  A merge of more than 128 partial rows is slow
-// (one kv head, 39,712 tokens: 46.9 and 28.3).
+// and 14.8; 8 x 1,000 with 1,024 22.0 and 31.6; 32 x 250 with 78 20.5 and 19.6.
+// A merge of more than 128 partial rows is slow (one kv head, 39,712 tokens:
+// 46.9 and 28.3).
 // A stream that the device counts may hold anything from none of its n_stream
 // rows to all: the cost at both ends counts, the tiles then for more, since the
 // workgroups planned for the extra tokens stand idle at first (planned for
-// 1,968, 68 there: 4 x 2,200 21.3 and 14.2, 1 x 8,124 13.9 and 13.5).
+// 1,968, 68 there: 4 x 2,200 16.5 and 14.2, 1 x 8,124 14.8 and 13.6).
 inline bool use_tok(const shard_decode_args* a) {
   if (a->kernel == 2) return true;
   if (a->kernel == 1) return !split_supported(a);

@@ -8,7 +8,7 @@
 //      twisted factorization.
 //   3. k_back, a wave per eigenvector: the reflectors applied in reverse.
 //
-// The vectors of eigenvalues closer than about 1e-6 of the largest one lose
+// The vectors of eigenvalues closer than about 1e-7 of the largest one lose
 // orthogonality in step 2 (no reorthogonalization): the caller checks V^T V and
 // the residual and takes a library routine where they miss its bound.
 #include "common.h"
@@ -52,9 +52,10 @@ __device__ __forceinline__ double wave_sum(double v) {
 // operations, cheaper than a second launch), then each wave updates one row
 // i > k with v w^T + w v^T and takes its product with the new reflector:
 // one launch, one pass over the trailing matrix, per column.  The last
-// workgroup, active to the end, writes d, e, tau and V's row k.  About 4 us a
-// launch at n = 1024, the launch itself and two block reductions; the matrix
-// (8 MB, read and written once a launch) stays in the last-level cache.
+// workgroup, active to the end, writes d, e, tau and V's row k.  5.2 us a launch
+// at n = 1024 (6.6 ms the whole solve; 5.9 traced with other work on the GPU), the
+// launch itself and two block reductions; the matrix (8 MB, read and written once
+// a launch) stays in the last-level cache.
 __global__ __launch_bounds__(256)
 void k_tridiag(double* __restrict__ A, int n, int k, const double* __restrict__ pin,
                double* __restrict__ pout, double* __restrict__ V, double* __restrict__ d,

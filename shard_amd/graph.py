@@ -19,7 +19,8 @@ eager decode step was masked) and transformers' Llama attention patched by
 tensors must keep their addresses: `reorder_cache` raises, and eager appends
 go through the graph's rows.  The graph keeps the shared decode workspace it
 captured alive.  The work plan of every captured call (its kernel choice and
-split balance) covers the stream rows of all `max_steps` steps from step 0.
+split balance) covers the stream rows of all `max_steps` steps from step 0; it
+weighs the stream both empty and full.
 """
 import torch
 
