@@ -1630,6 +1630,11 @@ inline bool split_supported(const shard_decode_args* a) {
          a->rank % 32 == 0 && a->rank <= 192 && n_extra(a) <= kMaxExtra;
 }
 
+// Workspace of a call with `parts` partial rows per query head.
+inline size_t partial_bytes(const shard_decode_args* a, int parts) {
+  return (size_t)a->batch * a->n_q_heads * parts * (kHD + 2) * sizeof(float);
+}
+
 // Row-split kernel: the workgroups of a (batch row, kv head).
 struct RowPlan {
   int n_t, n_xs, n_splits;  // tile splits, extra-token splits, both
@@ -1672,7 +1677,7 @@ inline RowPlan row_plan(const shard_decode_args* a) {
   w.n_t = tile_splits(w.n_xs);
   if (n_extra(a) <= kXFew && w.n_xs == n_pass) {
     const int n_xs = passes(kXShort);
-    if (tile_splits(n_xs) == w.n_t &&
+    if (tile_splits(n_xs) == w.n_t && w.n_t + n_xs <= std::max(room, w.n_t + 1) &&
         ceil_div((w.n_t + n_xs) * heads, cus) == ceil_div((w.n_t + w.n_xs) * heads, cus)) {
       w.x_wave = kXShort;
       w.n_xs = n_xs;
@@ -1776,6 +1781,10 @@ inline bool use_tok(const shard_decode_args* a) {
   const RowPlan row = row_plan(a);
   if (row.n_splits > 128) return true;
   const TokPlan tok = tok_plan(a);
+  // partial rows beyond the no-allocation scratch (two per head from 253 rows of
+  // 32 heads on, one tile each): the plan that writes fewer
+  if (partial_bytes(a, row.n_splits) > SHARD_DECODE_NOALLOC_SCRATCH_BYTES && tok.ns < row.n_splits)
+    return true;
   const int64_t wgs = (int64_t)tok.ns * a->n_kv_heads * a->batch;  // 4 query heads per kv head
   const int64_t later = (wgs - 1) / device_cus();                  // rounds after the first
   const int64_t tok_x = std::min(tok.n_xt, tok.per_u);
@@ -1907,11 +1916,7 @@ int shard_decode_supported(const shard_decode_args* a) {
 
 size_t shard_decode_attn_workspace(const shard_decode_args* a) {
   if (!a || a->batch <= 0 || a->n_q_heads <= 0 || a->n_comp <= 0 || !tok_supported(a)) return 0;
-  if (use_tok(a)) {
-    const TokPlan pl = tok_plan(a);
-    return (size_t)a->batch * a->n_q_heads * pl.ns * (kHD + 2) * sizeof(float);
-  }
-  return (size_t)a->batch * a->n_q_heads * row_plan(a).n_splits * (kHD + 2) * sizeof(float);
+  return partial_bytes(a, use_tok(a) ? tok_plan(a).ns : row_plan(a).n_splits);
 }
 
 }  // extern "C"

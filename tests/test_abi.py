@@ -150,6 +150,20 @@ def test_row_split_partial_rows_stay_within_the_chip(batch, n_comp, extra):
     assert need <= ops.DECODE_NOALLOC_SCRATCH_BYTES
 
 
+@pytest.mark.parametrize("batch,n_kv,n_comp,extra,n_splits,kernel", [
+    (16, 2, 4000, 68, 400, 1), (31, 2, 4000, 128, 64, 1),   # one row more than the tile splits
+    (256, 8, 1, 68, 0, 0), (400, 8, 32, 2048, 0, 0)])       # one tile per head: a single row
+def test_partial_rows_at_the_scratch_limit(batch, n_kv, n_comp, extra, n_splits, kernel):
+    """Calls whose partial rows just fit the no-allocation scratch fit it with
+    extra tokens too (host-only query)."""
+    from shard_amd import _lib, ops
+    a = _lib.DecodeArgs()
+    a.batch, a.n_q_heads, a.n_kv_heads, a.head_dim = batch, 4 * n_kv, n_kv, 128
+    a.rank, a.n_comp, a.n_splits, a.kernel = 192, n_comp, n_splits, kernel
+    a.n_sink, a.n_win, a.n_stream = 4, 64, extra - 68
+    assert 0 < _lib.load().shard_decode_attn_workspace(ctypes.byref(a)) <= ops.DECODE_NOALLOC_SCRATCH_BYTES
+
+
 @pytest.mark.parametrize("batch,n_kv,n_comp,extra,want,want_counted", [
     (1, 8, 1980, 132, 1, 1), (1, 8, 2000, 1968, 1, 1), (1, 8, 8124, 268, 1, 1),
     (1, 8, 12000, 78, 2, 2), (2, 8, 4400, 1968, 1, 1), (4, 8, 2200, 1968, 1, 2),
