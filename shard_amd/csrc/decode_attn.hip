@@ -432,6 +432,7 @@ __device__ __forceinline__ void decode_extras(const SplitParams& p, const int g,
 #pragma unroll
   for (int h = 0; h < kGQA; ++h) acc[h] = make_float2(0.f, 0.f);
   for (int x0 = xi * XT; x0 < n_x; x0 += p.n_xs * XT) {
+    const bool again = x0 >= p.n_xs * XT;  // a pass after the workgroup's first
     const bool mine = col < tw && x0 + tw * w + col < n_x;
     const int xt = min(x0 + tw * w + min(col, tw - 1), n_x - 1);  // clamped: other rows are masked
     int mpos;
@@ -467,7 +468,8 @@ __device__ __forceinline__ void decode_extras(const SplitParams& p, const int g,
         mx = fmaxf(mx, s[k]);
       }
       const float m_old = m_run;
-      m_run = fmaxf(m_old, wave64_reduce(mx, OpMax()));
+      m_run = wave64_reduce(mx, OpMax());
+      if (again) m_run = fmaxf(m_old, m_run);
       float ps = 0.f;
 #pragma unroll
       for (int k = 0; k < XV; ++k) {
@@ -476,12 +478,15 @@ __device__ __forceinline__ void decode_extras(const SplitParams& p, const int g,
         xpw[lane + 64 * k][w] = pk;
       }
       ps = wave64_reduce(ps, OpAdd());
-      const float al = m_run == -INFINITY ? 1.f : fast_exp2(m_old - m_run);
-      l_run = l_run * al + ps;
-      if (lane == 0) xal[w] = al;
+      if (again) {
+        const float al = m_run == -INFINITY ? 1.f : fast_exp2(m_old - m_run);
+        ps += l_run * al;
+        if (lane == 0) xal[w] = al;
+      }
+      l_run = ps;
     }
     __syncthreads();
-    if (x0 >= p.n_xs * XT) {  // a pass after the workgroup's first
+    if (again) {
 #pragma unroll
       for (int h = 0; h < kGQA; ++h) {
         acc[h].x *= xal[h];
